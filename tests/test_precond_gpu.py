@@ -91,6 +91,45 @@ def test_conv_forward_and_gradients(ks, cin, cout):
     assert float((got_dx - ref_dx).abs().max()) <= 1e-5 * float(ref_dx.abs().max())
 
 
+# tile edges of the convolution kernels (32 columns by 16, 8 or 4 rows, channel
+# blocks of 32 with a last one of 16, 64 output channels a workgroup where they
+# divide) and strides that allow 16-byte accesses or only 8-byte ones
+@pytest.mark.parametrize("cin,cout,H,W,pad", [
+    (16, 32, 1, 1, 0), (32, 64, 16, 32, 0), (48, 64, 17, 33, 4), (64, 64, 8, 31, 0), (96, 32, 15, 64, 8),
+    (64, 128, 9, 65, 4), (128, 16, 4, 5, 0), (80, 48, 33, 34, 12),
+])
+def test_conv3_tile_edges(cin, cout, H, W, pad):
+    from rang import precond as P
+
+    lib, st = P._lib(), P._stream()
+    g = torch.Generator().manual_seed(cin + cout + H + W)
+    B = 2
+    x = torch.randn(B * H * W, cin + pad, generator=g)
+    dy = torch.randn(B * H * W, cout + pad, generator=g)
+    w = torch.randn(cout, 9, cin, generator=g) / math.sqrt(9 * cin)
+    xb, wb, dyb = bf16_bits(x).cuda(), bf16_bits(w).cuda(), bf16_bits(dy).cuda()
+    y = torch.full((B * H * W, cout + pad), 7.0, device="cuda")
+    P._ok(lib.rang_amd_nn_conv_fwd(P._p(xb), cin + pad, pad, P._p(wb), P._p(y), None, cout + pad, pad, B, H, W, cin,
+                                   cout, 3, 0, st))
+    dw = torch.ones(cout, 9, cin, device="cuda")
+    P._ok(lib.rang_amd_nn_conv_wgrad(P._p(xb), cin + pad, pad, P._p(dyb), cout + pad, pad, P._p(dw), B, H, W, cin,
+                                     cout, 3, st))
+    xr = nchw(from_bits(xb.cpu())[:, pad:].contiguous(), B, H, W, cin).double()
+    dyr = nchw(from_bits(dyb.cpu())[:, pad:].contiguous(), B, H, W, cout).double()
+    wr = torch_weight(from_bits(wb.cpu()), 3).double()
+    ref = F.conv2d(xr, wr, padding=1)
+    got = nchw(y.cpu()[:, pad:].contiguous(), B, H, W, cout).double()
+    # FP32 sums of 9 cin (forward) and B H W (gradient) exact products: each
+    # addition rounds by 2^-24 of the sum of magnitudes
+    bound = 9 * cin * 2.0 ** -24 * float(F.conv2d(xr.abs(), wr.abs(), padding=1).max())
+    assert float((got - ref).abs().max()) <= bound
+    assert bool((y.cpu()[:, :pad] == 7.0).all())  # channels beside the output are left alone
+    ref_dw = torch.nn.grad.conv2d_weight(xr, wr.shape, dyr, padding=1) + 1.0
+    bound = (B * H * W + 1) * 2.0 ** -24 * float(
+        torch.nn.grad.conv2d_weight(xr.abs(), wr.shape, dyr.abs(), padding=1).max() + 1.0)
+    assert float((torch_weight(dw.cpu(), 3).double() - ref_dw).abs().max()) <= bound
+
+
 def test_pool_and_upsample_with_gradients():
     from rang import precond as P
 
