@@ -130,6 +130,41 @@ def test_conv3_tile_edges(cin, cout, H, W, pad):
     assert float((torch_weight(dw.cpu(), 3).double() - ref_dw).abs().max()) <= bound
 
 
+# eight channels a thread (16, 0), or one where the stride (pad 2) or the channel
+# count does not allow it
+@pytest.mark.parametrize("C,pad", [(16, 0), (24, 8), (16, 2), (12, 0)])
+def test_resampling_widths(C, pad):
+    from rang import precond as P
+
+    lib, st = P._lib(), P._stream()
+    g = torch.Generator().manual_seed(C + pad)
+    B, H, W, ld = 2, 6, 10, C + pad
+    x = bf16_bits(torch.randn(B * H * W, ld, generator=g)).cuda()
+    small = torch.full((B * H * W // 4, ld), 5, dtype=torch.int16, device="cuda")
+    P._ok(lib.rang_amd_nn_pool(P._p(x), ld, pad, P._p(small), ld, pad, B, H, W, C, st))
+    xr = nchw(from_bits(x.cpu())[:, pad:].contiguous(), B, H, W, C)
+    # four BF16 values summed in FP32 in their order, a quarter, rounded to BF16
+    q = ((xr[..., 0::2, 0::2] + xr[..., 0::2, 1::2]) + xr[..., 1::2, 0::2]) + xr[..., 1::2, 1::2]
+    assert torch.equal(nchw(small.cpu()[:, pad:].contiguous(), B, H // 2, W // 2, C), bf16_bits(0.25 * q))
+    assert bool((small.cpu()[:, :pad] == 5).all())
+    up = torch.full((B * H * W, ld), 5, dtype=torch.int16, device="cuda")
+    P._ok(lib.rang_amd_nn_up(P._p(small), ld, pad, P._p(up), ld, pad, B, H, W, C, st))
+    s = nchw(small.cpu()[:, pad:].contiguous(), B, H // 2, W // 2, C)
+    assert torch.equal(nchw(up.cpu()[:, pad:].contiguous(), B, H, W, C),
+                       s.repeat_interleave(2, 2).repeat_interleave(2, 3))
+    gy, gx = torch.randn(B * H * W // 4, ld, generator=g), torch.randn(B * H * W, ld, generator=g)
+    dgx = gx.cuda()
+    P._ok(lib.rang_amd_nn_pool_bwd(P._p(gy.cuda()), ld, pad, P._p(dgx), ld, pad, B, H, W, C, st))
+    ref = nchw(gx[:, pad:].contiguous(), B, H, W, C) + 0.25 * nchw(gy[:, pad:].contiguous(), B, H // 2, W // 2, C
+                                                                  ).repeat_interleave(2, 2).repeat_interleave(2, 3)
+    assert float((nchw(dgx.cpu()[:, pad:].contiguous(), B, H, W, C) - ref).abs().max()) <= 2.0 ** -22 * 8
+    back = torch.zeros(B * H * W // 4, ld, device="cuda")
+    P._ok(lib.rang_amd_nn_up_bwd(P._p(gx.cuda()), ld, pad, P._p(back), ld, pad, B, H, W, C, st))
+    gr = nchw(gx[:, pad:].contiguous(), B, H, W, C)
+    ref = ((gr[..., 0::2, 0::2] + gr[..., 0::2, 1::2]) + gr[..., 1::2, 0::2]) + gr[..., 1::2, 1::2]
+    assert torch.equal(nchw(back.cpu()[:, pad:].contiguous(), B, H // 2, W // 2, C), ref)
+
+
 def test_pool_and_upsample_with_gradients():
     from rang import precond as P
 
