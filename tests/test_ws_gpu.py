@@ -213,3 +213,23 @@ def test_wide_field_8192_pads_to_a_side_with_a_large_prime():
     assert (x, y) == (w // 2 - 300, w // 2 - 200)
     assert abs(psf[w // 2, w // 2] - 1.0) <= 1e-12
     assert abs(dirty[y, x] - 1.0) < 0.05
+
+
+# the tiled gridding at its edges: grids of one tile that wrap onto themselves
+# (8 x 12), last tiles of ks - 1 cells and of odd width, kernels of other
+# sizes, a grid below the kernel and a kernel above a tile (both gridded
+# without tiles), and tiles split over several items (5000 rows near u = v = 0)
+@pytest.mark.parametrize("width,height,ks,nrow,precision", [
+    (8, 12, 7, 300, "f64"), (36, 32, 7, 300, "f64"), (44, 100, 7, 300, "f32"), (64, 40, 3, 300, "f64"),
+    (60, 88, 9, 300, "f64"), (40, 36, 15, 300, "f64"), (4, 4, 7, 200, "f64"), (64, 64, 33, 60, "f64"),
+    (48, 48, 7, 5000, "f64"), (48, 48, 7, 5000, "f32"),
+])
+def test_tiled_gridding_edges(width, height, ks, nrow, precision):
+    c = survey_case(seed=width + ks, nrow=nrow, nchan=3, width=width, height=height, w_layers=3)
+    if nrow == 5000:
+        c["uvw"][:, :2] *= 0.05
+    r = gpu(c, precision, kernel_size=ks, oversampling=63, padding=1.0)
+    ref = oracle(c, kernel_size=ks, oversampling=63, padding=1.0)
+    assert rel(r["dirty"], ref["dirty"]) < TOL[precision]
+    assert rel(r["psf"], ref["psf"]) < TOL[precision]
+    same_stats(r["stats"], ref["stats"], precision)
