@@ -372,6 +372,11 @@ struct Geo {
     int mfma;
 };
 
+// Width in u and v of a tile: the matrix-core gridding's last tiles may be
+// partial (every other tiling divides the grid).
+__device__ __forceinline__ int tile_wu(const Geo& g, int tu) { return min(g.Tu, g.nu - tu * g.Tu); }
+__device__ __forceinline__ int tile_wv(const Geo& g, int tv) { return min(g.Tv, g.nv - tv * g.Tv); }
+
 __device__ __forceinline__ int upos(const Geo& g, int u) { return g.lu1 ? (u % g.lu1) * g.lu2 + u / g.lu1 : u; }
 __device__ __forceinline__ int vpos(const Geo& g, int v) { return g.lv1 ? (v % g.lv1) * g.lv2 + v / g.lv1 : v; }
 
@@ -602,7 +607,7 @@ __device__ __forceinline__ std::uint32_t key_of(const DevIn& in, const Geo& g, u
     const int su = shifted(iu0, g.nu), sv = shifted(iv0, g.nv);
     const int tu = su / g.Tu, tv = sv / g.Tv;
     const int ou = su - tu * g.Tu, ov = sv - tv * g.Tv;
-    const int cat = ((ou + g.supp > g.Tu) ? 2 : 0) | ((ov + g.supp > g.Tv) ? 1 : 0);
+    const int cat = ((ou + g.supp > tile_wu(g, tu)) ? 2 : 0) | ((ov + g.supp > tile_wv(g, tv)) ? 1 : 0);
     return std::uint32_t((((long long)tu * g.ntv + tv) * 4 + cat) * g.nb + minplane(g, w));
 }
 
@@ -957,13 +962,14 @@ __global__ __launch_bounds__(256) void k_zero_split(Geo g, const std::uint32_t* 
     // a fixed column per thread, rows in steps (no division per cell)
     const int istep = int(blockDim.x) / g.Tv;
     const int i0 = int(threadIdx.x) / g.Tv, j = int(threadIdx.x) - i0 * g.Tv;
-    if (i0 >= istep) return;
+    const int wu = tile_wu(g, tu);
+    if (i0 >= istep || j >= tile_wv(g, tv)) return;
     int gcol = tv * g.Tv + j + g.nv / 2;
     if (gcol >= g.nv) gcol -= g.nv;
     for (int o = 0; o < NOUT; ++o)
         for (int pl = 0; pl < np; ++pl) {
             cx<T>* base = grid + (long long)o * P * plane + (long long)(p0 + pl) * plane + gcol;
-            for (int i = i0; i < g.Tu; i += istep) {
+            for (int i = i0; i < wu; i += istep) {
                 int grow = tu * g.Tu + i + g.nu / 2;
                 if (grow >= g.nu) grow -= g.nu;
                 base[(long long)grow * g.nv] = cx<T>{T(0), T(0)};
@@ -1048,7 +1054,7 @@ template <class T>
 __device__ __forceinline__ Rec<T> grid_fetch(const Geo& g, const Rec<T>* __restrict__ recs,
                                              const std::uint32_t* s_start,
                                              const std::uint32_t* s_pre, std::uint32_t j, int p0,
-                                             int p1, const cx<T>* __restrict__ stored) {
+                                             int p1, int tu, int tv, const cx<T>* __restrict__ stored) {
     int src = 0;
     while (j >= s_pre[src + 1]) ++src;
     const std::uint32_t at = s_start[src] + (j - s_pre[src]);
@@ -1063,8 +1069,9 @@ __device__ __forceinline__ Rec<T> grid_fetch(const Geo& g, const Rec<T>* __restr
     }
     int du, dv, cat;
     source_of(src, du, dv, cat);
-    const int ou = int(r.pos & 255u) - (du ? g.Tu : 0) + 64;
-    const int ov = int((r.pos >> 8) & 255u) - (dv ? g.Tv : 0) + 64;
+    // the tile before is the grid's last one (perhaps partial) for tile 0
+    const int ou = int(r.pos & 255u) - (du ? (tu ? g.Tu : tile_wu(g, g.ntu - 1)) : 0) + 64;
+    const int ov = int((r.pos >> 8) & 255u) - (dv ? (tv ? g.Tv : tile_wv(g, g.ntv - 1)) : 0) + 64;
     const int mp = int(r.pos >> 16);
     r.pos = std::uint32_t(ou) | (std::uint32_t(ov) << 8);
     if (g.wgrid) {
@@ -1171,14 +1178,14 @@ __device__ __forceinline__ void grid_item(Geo g, const Rec<T>* __restrict__ recs
     Rec<T> nxt{};
     const cx<T>* stored = static_cast<const cx<T>*>(in.stored);
     if (stager && jbeg + threadIdx.x < jend)
-        nxt = grid_fetch(g, recs, s_start, s_pre, jbeg + threadIdx.x, p0, p1, stored);
+        nxt = grid_fetch(g, recs, s_start, s_pre, jbeg + threadIdx.x, p0, p1, tu, tv, stored);
     for (std::uint32_t base = jbeg; base < jend; base += kGridBatch) {
         const int nbat = int(min(jend - base, std::uint32_t(kGridBatch)));
         __syncthreads();  // the previous batch is consumed
         if (int(threadIdx.x) < nbat) s_rec[threadIdx.x] = nxt;
         __syncthreads();
         const std::uint32_t jn = base + kGridBatch + threadIdx.x;
-        if (stager && jn < jend) nxt = grid_fetch(g, recs, s_start, s_pre, jn, p0, p1, stored);
+        if (stager && jn < jend) nxt = grid_fetch(g, recs, s_start, s_pre, jn, p0, p1, tu, tv, stored);
         if constexpr (REG && RPW == 1) {
             if (g.wgrid) {
                 // One visibility per wave: its position is wave-uniform, and
@@ -1418,21 +1425,27 @@ __global__ __launch_bounds__(grid_threads<T>()) void k_grid_jobs(const GridJob<T
 
 // ------------------------------------------------------------ gridding on the matrix cores
 
-// Single-precision w-gridding on 16 x 16 tiles with the matrix cores: one
-// wave per item (tile, group of up to kMfmaPlanes planes, chunk), whose
-// accumulators are the item's planes of the tile held in the MFMA result
-// registers, so that no LDS atomics are needed. Four visibilities at a
-// time: with A[i][k] = ku_k(i - ou_k) kw_k(plane) (lane 16 k + i) and
-// B[k][j] = kv_k(j - ov_k) v_k (lane 16 k + j), one
-// v_mfma_f32_16x16x4_f32 per plane and part adds sum_k A[i][k] B[k][j] to
-// cell (i, j) of the plane, which is the gridding sum (wgridder.rs:2098-2156)
-// for those four visibilities; taps outside a visibility's footprint or
-// planes are zero. Lane 16 k + t evaluates tap t of visibility k at its u,
-// v and w arguments once; the operands fetch theirs across lanes. The
-// result register r of lane l holds cell (4 (l / 16) + r, l mod 16).
-// Planes per item and the occupancy target, measured on the 464M workload
-// (gridding stage): 8 planes at 4 waves per SIMD 103.5 ms (117.4 without the
-// target), 6 at 5 waves 105.9, 4 at 6 waves 111.4.
+// W-gridding on 16 x 16 windows with the matrix cores: one wave per item
+// (tile, group of planes, chunk), whose accumulators are the item's planes of
+// the tile held in the MFMA result registers, so that no LDS atomics are
+// needed. Four visibilities at a time: with A[i][k] = ku_k(i - ou_k) kw_k(plane)
+// (lane 16 k + i) and B[k][j] = kv_k(j - ov_k) v_k (lane 16 k + j), one
+// v_mfma_f32_16x16x4_f32 or v_mfma_f64_16x16x4_f64 per plane and part adds
+// sum_k A[i][k] B[k][j] to cell (i, j) of the plane, which is the gridding sum
+// (wgridder.rs:2098-2156) for those four visibilities; taps outside a
+// visibility's footprint or planes are zero. Lane 16 k + t evaluates tap t of
+// visibility k once; the operands fetch theirs across lanes. In result
+// register r lane l holds column l mod 16 of row 4 (l / 16) + r in single and
+// (l / 16) + 4 r in double precision.
+//
+// Single precision, measured on the 464M workload (gridding stage): 8 planes
+// at 4 waves per SIMD 103.5 ms (117.4 without the target), 6 at 5 waves 105.9,
+// 4 at 6 waves 111.4. Double precision: the LDS gridder is bound by its
+// double LDS adds (2 S^3 a visibility and output at 5.5 a clock and CU); 16 x
+// 16 x 4 products of 64 clocks take a third of that. 23.8 M visibilities,
+// dirty and PSF, support 7 (7 planes): the call 43.9 -> 17.4 ms, eight planes
+// an item at one wave per SIMD (256 registers of accumulators); four planes at
+// two waves 19.1, five 20.2. Support 11, 118 k visibilities: 720 -> 195 us.
 constexpr int kMfmaPlanes = 8;
 
 // Lane q of each row of 16 lanes, broadcast to its row (DPP row_newbcast;
@@ -1450,27 +1463,57 @@ __device__ __forceinline__ int row_bcast(int v, int q) {
     }
 }
 static_assert(kMfmaPlanes <= 8, "row_bcast covers planes 0-7");
+__device__ __forceinline__ float row_bcast(float v, int q) { return __int_as_float(row_bcast(__float_as_int(v), q)); }
+__device__ __forceinline__ double row_bcast(double v, int q) {
+    const long long b = __double_as_longlong(v);
+    const unsigned lo = unsigned(row_bcast(int(b), q)), hi = unsigned(row_bcast(int(b >> 32), q));
+    return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
+}
+
 constexpr int kMfmaTile = 16;
 typedef float mfma_v4 __attribute__((ext_vector_type(4)));
+typedef double mfma_d4 __attribute__((ext_vector_type(4)));
 
-template <int S>
+template <class T>
+struct Mfma;
+template <>
+struct Mfma<float> {
+    using Acc = mfma_v4;
+    static __device__ __forceinline__ Acc mul(float a, float b, Acc c) {
+        return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+    }
+    static __device__ __forceinline__ int row(int k, int r) { return 4 * k + r; }
+};
+template <>
+struct Mfma<double> {
+    using Acc = mfma_d4;
+    static __device__ __forceinline__ Acc mul(double a, double b, Acc c) {
+        return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
+    }
+    static __device__ __forceinline__ int row(int k, int r) { return k + 4 * r; }
+};
+
+template <class T, int S, int NOUT>
 struct MfmaShared {
-    float coef[2 * ne_of<S>() * S];
+    T coef[2 * ne_of<S>() * S];
     std::uint32_t start[9], pre[10];
-    Rec<float> rec[64];
+    Rec<T> rec[64];
+    cx<T> unit[NOUT == 2 ? 64 : 1];  // the second output's values
     int qr[32];  // per group of 4 staged records: its planes [lo, hi) in the item
 };
 
-template <int S, bool FORM>
-__device__ __forceinline__ void grid_item_mfma(Geo g, const Rec<float>* __restrict__ recs,
+template <class T, int S, int NOUT, bool FORM>
+__device__ __forceinline__ void grid_item_mfma(Geo g, const Rec<T>* __restrict__ recs,
                                                const std::uint32_t* __restrict__ off,
-                                               const float* __restrict__ coeff, DevIn in, int G, int ngroups,
+                                               const T* __restrict__ coeff, DevIn in, int G, int ngroups,
                                                std::uint32_t rc, const std::uint32_t* __restrict__ item_off,
                                                const std::uint32_t* __restrict__ order,
-                                               cx<float>* __restrict__ grid, std::uint32_t item, float* coef,
-                                               std::uint32_t* s_start, std::uint32_t* s_pre, Rec<float>* s_rec,
-                                               int* s_qr) {
-    constexpr int NE = ne_of<S>();
+                                               cx<T>* __restrict__ grid, std::uint32_t item, T* coef,
+                                               std::uint32_t* s_start, std::uint32_t* s_pre, Rec<T>* s_rec,
+                                               cx<T>* s_unit, int* s_qr) {
+    using M = Mfma<T>;
+    using Acc = typename M::Acc;
+    constexpr int NE = ne_of<S>(), KP = kMfmaPlanes;
     const int lane = threadIdx.x;
     const int ntg = g.ntu * g.ntv * ngroups;
     int tg;
@@ -1497,47 +1540,54 @@ __device__ __forceinline__ void grid_item_mfma(Geo g, const Rec<float>* __restri
     __syncthreads();
     const std::uint32_t jbeg = chunk * rc, jend = min(s_pre[9], jbeg + rc);
     const int k = lane >> 4, i = lane & 15;
-    // lane 16 k + i holds tap i (u and w) for i < S and tap i - S (v) for
-    // S <= i < 2 S of visibility k: the u and v taps in one evaluation
-    static_assert(2 * S <= 16, "u and v taps share a row of 16 lanes");
+    // up to support 8, lane 16 k + i holds tap i (u and w) for i < S and tap
+    // i - S (v) for S <= i < 2 S of visibility k: the u and v taps in one
+    // evaluation; beyond, tap i of each
+    constexpr bool PAIR = 2 * S <= 16;
     const bool lane_u = i < S;
-    TapReg<float, S> tr;
-    tr.load(coef, lane_u ? i : min(i - S, S - 1));
-    const cx<float>* stored = static_cast<const cx<float>*>(in.stored);
-    mfma_v4 are[kMfmaPlanes], aim[kMfmaPlanes];
+    TapReg<T, S> tr;
+    tr.load(coef, lane_u ? i : PAIR ? min(i - S, S - 1) : S - 1);
+    // the lane's row and column lie in the tile (the last tiles may be partial)
+    const int wu = tile_wu(g, tu), wv = tile_wv(g, tv);
+    const cx<T>* stored = static_cast<const cx<T>*>(in.stored);
+    Acc are[NOUT][KP], aim[NOUT][KP];
 #pragma unroll
-    for (int q = 0; q < kMfmaPlanes; ++q) {
-        are[q] = mfma_v4{0.f, 0.f, 0.f, 0.f};
-        aim[q] = mfma_v4{0.f, 0.f, 0.f, 0.f};
-    }
+    for (int o = 0; o < NOUT; ++o)
+#pragma unroll
+        for (int q = 0; q < KP; ++q) are[o][q] = aim[o][q] = Acc{T(0), T(0), T(0), T(0)};
+    // the second output's imaginary part is zero without shifts
+    const bool unit_im = NOUT == 2 && g.shifting;
     for (std::uint32_t base = jbeg; base < jend; base += 64) {
         const int nrec = int(min(jend - base, 64u));
-        Rec<float> r{};
+        Rec<T> r{};
+        cx<T> unit{T(0), T(0)};
         if (lane < nrec) {
-            r = grid_fetch(g, recs, s_start, s_pre, base + lane, p0, p1, stored);
-            if constexpr (FORM) {
-                const float fl = (r.idx & kFlip) ? -1.f : 1.f;
-                const cx<float> d = cmul(vis_get<float>(in, r.idx & ~kFlip), cx<float>{r.re, r.im * fl});
+            r = grid_fetch(g, recs, s_start, s_pre, base + lane, p0, p1, tu, tv, stored);
+            if constexpr (FORM || NOUT == 2) {
+                unit = cx<T>{r.re, r.im};
+                const T fl = (r.idx & kFlip) ? T(-1) : T(1);
+                const cx<T> d = cmul(vis_get<T>(in, r.idx & ~kFlip), cx<T>{r.re, r.im * fl});
                 r.re = d.re;
                 r.im = d.im * fl;
             }
         } else {
             // no taps anywhere: offsets far outside the tile, an empty plane span
             r.pos = 0u;
-            r.re = r.im = 0.f;
+            r.re = r.im = T(0);
         }
         // the planes of each group of four records: the union of their
         // item planes, reduced over the four lanes once per batch
         {
             int tlo, thi, q0, mp;
             taps_on_item(r.pos, p0, tlo, thi, q0, mp);
-            int qa = thi > tlo ? q0 : kMfmaPlanes, qb = thi > tlo ? q0 + thi - tlo : 0;
+            int qa = thi > tlo ? q0 : KP, qb = thi > tlo ? q0 + thi - tlo : 0;
             qa = min(qa, __shfl_xor(qa, 1, 64));
             qb = max(qb, __shfl_xor(qb, 1, 64));
             qa = min(qa, __shfl_xor(qa, 2, 64));
             qb = max(qb, __shfl_xor(qb, 2, 64));
             __syncthreads();  // the previous batch is consumed
             s_rec[lane] = r;
+            if constexpr (NOUT == 2) s_unit[lane] = unit;
             if ((lane & 3) == 0) {
                 s_qr[lane >> 1] = qa;
                 s_qr[(lane >> 1) + 1] = min(qb, np);
@@ -1545,23 +1595,36 @@ __device__ __forceinline__ void grid_item_mfma(Geo g, const Rec<float>* __restri
         }
         __syncthreads();
         for (int g4 = 0; g4 < nrec; g4 += 4) {
-            const Rec<float>& rk = s_rec[g4 + k];
+            const Rec<T>& rk = s_rec[g4 + k];
             const std::uint32_t pos = rk.pos;
             const int ou = int(pos & 255u) - 64, ov = int((pos >> 8) & 255u) - 64;
             int tlo, thi, q0, mp;
             taps_on_item(pos, p0, tlo, thi, q0, mp);
-            const float tUV = tr.eval(lane_u ? rk.x0 : rk.y0);
+            T tU, tV;
+            if constexpr (PAIR) {
+                tU = tV = tr.eval(lane_u ? rk.x0 : rk.y0);
+            } else {
+                tU = tr.eval(rk.x0);
+                tV = tr.eval(rk.y0);
+            }
             // w taps zero on the lanes past the support: a fetch of tap t
             // of visibility k at lane 16 k + t for t in [-8, 16) then reads
-            // zero outside [0, S) (lane indices wrap modulo 64)
-            const float tW = lane_u ? tr.eval(warg_of(rk)) : 0.f;
+            // zero outside [0, S) (lane indices wrap modulo 64), up to support 8
+            const T tW = lane_u ? tr.eval(warg_of(rk)) : T(0);
             const int au = i - ou, av = i - ov;
-            const bool inu = au >= 0 && au < S, inv = av >= 0 && av < S;
-            const float ku = __shfl(tUV, 16 * k + (inu ? au : 0), 64);
-            const float kv = __shfl(tUV, 16 * k + S + (inv ? av : 0), 64);
-            const float A0 = inu ? ku : 0.f;
-            const float Bk = inv ? kv : 0.f;
-            const float bre = Bk * rk.re, bim = Bk * rk.im;
+            const bool inu = au >= 0 && au < S && i < wu, inv = av >= 0 && av < S && i < wv;
+            const T ku = __shfl(tU, 16 * k + (inu ? au : 0), 64);
+            const T kv = __shfl(tV, 16 * k + (PAIR ? S : 0) + (inv ? av : 0), 64);
+            const T A0 = inu ? ku : T(0);
+            const T Bk = inv ? kv : T(0);
+            T bre[NOUT], bim[NOUT];
+            bre[0] = Bk * rk.re;
+            bim[0] = Bk * rk.im;
+            if constexpr (NOUT == 2) {
+                const cx<T> u = s_unit[g4 + k];
+                bre[1] = Bk * u.re;
+                bim[1] = Bk * u.im;
+            }
             // the group's planes: the union of its visibilities' item planes
             const int qlo = __builtin_amdgcn_readfirstlane(s_qr[g4 >> 1]);
             const int qhi = __builtin_amdgcn_readfirstlane(s_qr[(g4 >> 1) + 1]);
@@ -1570,45 +1633,62 @@ __device__ __forceinline__ void grid_item_mfma(Geo g, const Rec<float>* __restri
             // on the item's other planes (q < q0 means tlo = 0; q past its
             // planes means thi = S or q >= np)
             // One permute per group puts the tap of plane j at lane 16 k + j
-            // (j < kMfmaPlanes); plane q then broadcasts lane q of each row of
+            // (j < KP); plane q then broadcasts lane q of each row of
             // 16 lanes (DPP row_newbcast, a register move on the VALU) instead
             // of waiting on a permute through the LDS per plane.
-            const int wbase = 4 * (16 * k + tlo - q0);
-            const int wq = __builtin_amdgcn_ds_bpermute(wbase + 4 * i, __float_as_int(tW));
+            T wq;
+            if constexpr (PAIR && sizeof(T) == 4) {
+                wq = __int_as_float(
+                    __builtin_amdgcn_ds_bpermute(4 * (16 * k + tlo - q0 + i), __float_as_int(tW)));
+            } else {
+                const int t = tlo - q0 + i;
+                const bool on = t >= 0 && t < S;
+                const T v = __shfl(tW, 16 * k + (on ? t : 0), 64);
+                wq = on ? v : T(0);
+            }
 #pragma unroll
-            for (int q = 0; q < kMfmaPlanes; ++q) {
+            for (int q = 0; q < KP; ++q) {
                 if (q < qlo || q >= qhi) continue;
-                const float kw = __int_as_float(row_bcast(wq, q));
-                const float a = A0 * kw;
-                are[q] = __builtin_amdgcn_mfma_f32_16x16x4f32(a, bre, are[q], 0, 0, 0);
-                aim[q] = __builtin_amdgcn_mfma_f32_16x16x4f32(a, bim, aim[q], 0, 0, 0);
+                const T a = A0 * row_bcast(wq, q);
+#pragma unroll
+                for (int o = 0; o < NOUT; ++o) {
+                    are[o][q] = M::mul(a, bre[o], are[o][q]);
+                    if (o == 0 || unit_im) aim[o][q] = M::mul(a, bim[o], aim[o][q]);
+                }
             }
         }
     }
-    // flush: register r of lane l is cell (4 (l / 16) + r, l mod 16)
+    // flush: column i of rows M::row(k, 0 .. 3), within the tile
+    if (i >= wv) return;
     const long long plane = (long long)g.nu * g.nv;
-    int gcol = tv * kMfmaTile + i + g.nv / 2;
+    int gcol = tv * g.Tv + i + g.nv / 2;
     if (gcol >= g.nv) gcol -= g.nv;
 #pragma unroll
-    for (int q = 0; q < kMfmaPlanes; ++q) {
-        if (q >= np) break;
-        cx<float>* dst = grid + (long long)(p0 + q) * plane + gcol;
+    for (int o = 0; o < NOUT; ++o)
 #pragma unroll
-        for (int rr = 0; rr < 4; ++rr) {
-            int grow = tu * kMfmaTile + 4 * k + rr + g.nu / 2;
-            if (grow >= g.nu) grow -= g.nu;
-            const float vre = are[q][rr], vim = aim[q][rr];
-            cx<float>* c = dst + (long long)grow * g.nv;
-            if (nchunks == 1) {
-                *c = cx<float>{vre, vim};
-            } else if (vre != 0.f || vim != 0.f) {
-                atomicAdd(&c->re, vre);
-                atomicAdd(&c->im, vim);
+        for (int q = 0; q < KP; ++q) {
+            if (q >= np) break;
+            cx<T>* dst = grid + ((long long)o * P + p0 + q) * plane + gcol;
+#pragma unroll
+            for (int rr = 0; rr < 4; ++rr) {
+                const int ti = M::row(k, rr);
+                if (ti >= wu) continue;
+                int grow = tu * g.Tu + ti + g.nu / 2;
+                if (grow >= g.nu) grow -= g.nu;
+                const T vre = are[o][q][rr], vim = aim[o][q][rr];
+                cx<T>* c = dst + (long long)grow * g.nv;
+                if (nchunks == 1) {
+                    *c = cx<T>{vre, vim};
+                } else if (vre != T(0) || vim != T(0)) {
+                    atomicAdd(&c->re, vre);
+                    atomicAdd(&c->im, vim);
+                }
             }
         }
-    }
 }
 
+// Waves per SIMD: four in single precision with one output (106 registers);
+// two where the accumulators take 128, one where they take 256.
 template <int S, bool FORM>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4, 8))) void k_grid_mfma(Geo g, const Rec<float>* __restrict__ recs,
                                                   const std::uint32_t* __restrict__ off,
@@ -1617,16 +1697,29 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4, 8))) void
                                                   const std::uint32_t* __restrict__ item_off,
                                                   const std::uint32_t* __restrict__ order,
                                                   cx<float>* __restrict__ grid) {
-    __shared__ MfmaShared<S> sh;
-    grid_item_mfma<S, FORM>(g, recs, off, coeff, in, G, ngroups, rc, item_off, order, grid, blockIdx.x, sh.coef,
-                            sh.start, sh.pre, sh.rec, sh.qr);
+    __shared__ MfmaShared<float, S, 1> sh;
+    grid_item_mfma<float, S, 1, FORM>(g, recs, off, coeff, in, G, ngroups, rc, item_off, order, grid, blockIdx.x,
+                                      sh.coef, sh.start, sh.pre, sh.rec, sh.unit, sh.qr);
+}
+
+template <class T, int S, int NOUT, bool FORM>
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 8 && NOUT == 2 ? 1 : 2, 4))) void k_grid_mfma_wide(Geo g, const Rec<T>* __restrict__ recs,
+                                                  const std::uint32_t* __restrict__ off,
+                                                  const T* __restrict__ coeff, DevIn in, int G,
+                                                  int ngroups, std::uint32_t rc,
+                                                  const std::uint32_t* __restrict__ item_off,
+                                                  const std::uint32_t* __restrict__ order,
+                                                  cx<T>* __restrict__ grid) {
+    __shared__ MfmaShared<T, S, NOUT> sh;
+    grid_item_mfma<T, S, NOUT, FORM>(g, recs, off, coeff, in, G, ngroups, rc, item_off, order, grid, blockIdx.x,
+                                     sh.coef, sh.start, sh.pre, sh.rec, sh.unit, sh.qr);
 }
 
 // Every job's items in one launch on the matrix cores (jobs as k_grid_jobs,
-// each gridded by k_grid_mfma's item body at its support).
+// each gridded by the item body above at its support).
 template <bool FORM>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4, 8))) void k_grid_mfma_jobs(const GridJob<float>* __restrict__ jobs, int njobs) {
-    __shared__ MfmaShared<8> sh;
+    __shared__ MfmaShared<float, 8, 1> sh;
     int j = 0;
     for (int k = 1; k < njobs; ++k)
         if (jobs[k].first <= blockIdx.x) j = k;
@@ -1635,15 +1728,29 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4, 8))) void
     switch (J.g.supp) {
 #define MJOB_CASE(SS)                                                                                    \
     case SS:                                                                                             \
-        grid_item_mfma<SS, FORM>(J.g, J.recs, J.off, J.coeff, J.in, J.G, J.ngroups, J.rc, J.item_off,    \
-                                 J.order, J.grid, item, sh.coef, sh.start, sh.pre, sh.rec, sh.qr);       \
+        grid_item_mfma<float, SS, 1, FORM>(J.g, J.recs, J.off, J.coeff, J.in, J.G, J.ngroups, J.rc, J.item_off, \
+                                 J.order, J.grid, item, sh.coef, sh.start, sh.pre, sh.rec, sh.unit, sh.qr); \
         break;
         MJOB_CASE(4) MJOB_CASE(5) MJOB_CASE(6) MJOB_CASE(7) MJOB_CASE(8)
-#undef MJOB_CASE
     default:
         break;
     }
 }
+
+// Double precision, one launch per support (its kernels differ too much in
+// registers to share one): the jobs of support S.
+template <int S>
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 4))) void k_grid_mfma_jobs64(const GridJob<double>* __restrict__ jobs, int njobs) {
+    __shared__ MfmaShared<double, S, 1> sh;
+    int j = 0;
+    for (int k = 1; k < njobs; ++k)
+        if (jobs[k].first <= blockIdx.x) j = k;
+    const GridJob<double>& J = jobs[j];
+    grid_item_mfma<double, S, 1, false>(J.g, J.recs, J.off, J.coeff, J.in, J.G, J.ngroups, J.rc, J.item_off, J.order,
+                                        J.grid, blockIdx.x - J.first, sh.coef, sh.start, sh.pre, sh.rec, sh.unit,
+                                        sh.qr);
+}
+#undef MJOB_CASE
 
 // ------------------------------------------------------------ transforms
 
@@ -2696,25 +2803,56 @@ void launch_grid(int S, int nblocks, std::size_t lds, hipStream_t st, const Geo&
     HIPCHK(hipGetLastError());
 }
 
-void launch_grid_mfma(int S, int nblocks, bool form, hipStream_t st, const Geo& g, const Rec<float>* recs,
-                      const std::uint32_t* off, const float* coeff, const DevIn& in, int G, int ngroups,
+template <class T>
+void launch_grid_mfma(int S, int nblocks, int nout, bool form, hipStream_t st, const Geo& g, const Rec<T>* recs,
+                      const std::uint32_t* off, const T* coeff, const DevIn& in, int G, int ngroups,
                       std::uint32_t rc, const std::uint32_t* item_off, const std::uint32_t* order,
-                      cx<float>* out) {
-#define MFMA_CASE(SS)                                                                                   \
-    case SS:                                                                                            \
-        if (form)                                                                                       \
-            k_grid_mfma<SS, true><<<nblocks, 64, 0, st>>>(g, recs, off, coeff, in, G, ngroups, rc, item_off, \
-                                                          order, out);                                  \
-        else                                                                                            \
-            k_grid_mfma<SS, false><<<nblocks, 64, 0, st>>>(g, recs, off, coeff, in, G, ngroups, rc, item_off, \
-                                                           order, out);                                 \
+                      cx<T>* out) {
+#define MFMA_LAUNCH(KERNEL) \
+    KERNEL<<<nblocks, 64, 0, st>>>(g, recs, off, coeff, in, G, ngroups, rc, item_off, order, out)
+#define MFMA_CASE(SS)                                                                      \
+    case SS:                                                                               \
+        if constexpr (SS <= max_support<T>()) {                                            \
+            if (nout == 2) {                                                               \
+                MFMA_LAUNCH((k_grid_mfma_wide<T, SS, 2, false>));                          \
+            } else if constexpr (sizeof(T) == 4) {                                         \
+                if (form)                                                                  \
+                    MFMA_LAUNCH((k_grid_mfma<SS, true>));                                  \
+                else                                                                       \
+                    MFMA_LAUNCH((k_grid_mfma<SS, false>));                                 \
+            } else {                                                                       \
+                if (form)                                                                  \
+                    MFMA_LAUNCH((k_grid_mfma_wide<T, SS, 1, true>));                       \
+                else                                                                       \
+                    MFMA_LAUNCH((k_grid_mfma_wide<T, SS, 1, false>));                      \
+            }                                                                              \
+        } else {                                                                           \
+            throw DevError{"kernel support too large for this precision"};                 \
+        }                                                                                  \
         break;
     switch (S) {
-        MFMA_CASE(4) MFMA_CASE(5) MFMA_CASE(6) MFMA_CASE(7) MFMA_CASE(8)
+        MFMA_CASE(4) MFMA_CASE(5) MFMA_CASE(6) MFMA_CASE(7) MFMA_CASE(8) MFMA_CASE(9) MFMA_CASE(10) MFMA_CASE(11)
+        MFMA_CASE(12) MFMA_CASE(13) MFMA_CASE(14) MFMA_CASE(15) MFMA_CASE(16)
     default:
         throw DevError{"unsupported kernel support"};
     }
 #undef MFMA_CASE
+#undef MFMA_LAUNCH
+    HIPCHK(hipGetLastError());
+}
+
+void launch_jobs64(int S, int nblocks, hipStream_t st, const GridJob<double>* jobs, int njobs) {
+#define JOB64_CASE(SS)                                              \
+    case SS:                                                        \
+        k_grid_mfma_jobs64<SS><<<nblocks, 64, 0, st>>>(jobs, njobs); \
+        break;
+    switch (S) {
+        JOB64_CASE(4) JOB64_CASE(5) JOB64_CASE(6) JOB64_CASE(7) JOB64_CASE(8) JOB64_CASE(9) JOB64_CASE(10)
+        JOB64_CASE(11) JOB64_CASE(12) JOB64_CASE(13) JOB64_CASE(14) JOB64_CASE(15) JOB64_CASE(16)
+    default:
+        throw DevError{"unsupported kernel support"};
+    }
+#undef JOB64_CASE
     HIPCHK(hipGetLastError());
 }
 
@@ -2755,6 +2893,15 @@ int choose_tile(int n, int supp, int hi, int target) {
     for (int t = std::max(supp, 8); best < 0 && t <= std::min(64, n); ++t)
         if (n % t == 0) best = t;
     return best;
+}
+
+// Tile side of the matrix-core gridding on an axis of n cells: the largest up
+// to its 16-cell window whose last tile is whole or at least supp - 1 cells (a
+// footprint then reaches at most the next tile), 0 where there is none.
+int mfma_tile(int n, int supp) {
+    for (int t = kMfmaTile; t >= std::max(12, supp - 1); --t)
+        if (n >= kMfmaTile && (n % t == 0 || n % t >= supp - 1)) return t;
+    return 0;
 }
 
 void exclusive_scan(Workspace& ws, const std::uint32_t* in, std::uint32_t* out, long long n,
@@ -2966,6 +3113,18 @@ constexpr std::size_t grid_lds() {
 // once a split tile's chunks add only the cells they reach (gridding stage:
 // 512 -> 280.5 ms, 1024 -> 251.6, 2048 -> 238.0, 4096 -> 233.4, 8192 -> 234.5).
 constexpr std::uint32_t kGridChunk = 4096;
+// On the matrix cores an item is one wave's serial work, so a call of few
+// visibilities takes shorter ones: about kGridItems items over the whole call
+// (a visibility reaches two to four tiles' items), at least 128 records each.
+// Measured, items of 4096 records -> this rule: 118 k visibilities 545 -> 365
+// us (single precision, host arrays) and 1594 -> 1350 us (normal operator,
+// double precision), 3.2 M 1448 -> 1255 us; twice or half as many items are
+// within 3 % of it, four times as many slower (3.2 M: 1520 us).
+constexpr long long kGridItems = 16384;
+std::uint32_t grid_chunk(const Geo& g) {
+    if (!g.mfma) return kGridChunk;
+    return std::uint32_t(std::max<long long>(128, std::min<long long>(kGridChunk, 4 * g.n / kGridItems)));
+}
 constexpr std::uint32_t kDegridChunk = 1024;     // visibilities per degridding item
 // Staged degridding holds a tile and its halo on every plane in LDS: in
 // single precision one 1024-thread workgroup per CU with up to 150 KiB and
@@ -3073,7 +3232,7 @@ bool mfma_enabled() {
 }
 
 template <class T>
-bool fill_geo(const Geometry& G, Geo& g, int nout, bool degrid, std::string& err, int tile = 0) {
+bool fill_geo(const Geometry& G, Geo& g, int nout, bool degrid, std::string& err, int tile = 0, bool fixed = false) {
     g.nx = int(G.nx);
     g.ny = int(G.ny);
     g.nu = int(G.nu);
@@ -3113,20 +3272,28 @@ bool fill_geo(const Geometry& G, Geo& g, int nout, bool degrid, std::string& err
     } else if (tile > 0) {
         target = std::min(tile, hi);  // the tuner's tile side
     }
-    // single-precision w-gridding of one image on 16 x 16 tiles on the
-    // matrix cores, unless a tile side is asked for
-    g.mfma = (sizeof(T) == 4 && !degrid && nout == 1 && g.wgrid && g.supp <= 8 && tile == 0 &&
-              g.nu % kMfmaTile == 0 && g.nv % kMfmaTile == 0 && mfma_enabled())
-                 ? 1
-                 : 0;
-    g.Tu = g.mfma ? kMfmaTile : choose_tile(g.nu, g.supp, std::min(hi, 64), target);
-    g.Tv = g.mfma ? kMfmaTile : choose_tile(g.nv, g.supp, std::min(hi, 64), target);
+    g.Tu = choose_tile(g.nu, g.supp, std::min(hi, 64), target);
+    g.Tv = choose_tile(g.nv, g.supp, std::min(hi, 64), target);
     if (g.Tu < 0 || g.Tv < 0) {
         err = "no tile size divides the grid";
         return false;
     }
-    g.ntu = g.nu / g.Tu;
-    g.ntv = g.nv / g.Tv;
+    // w-gridding goes to the matrix cores where the axes tile for them,
+    // unless a tile side is asked for (measured against the LDS gridder:
+    // 3.2 M visibilities, support 6, single precision 1227 -> 517 us; double
+    // precision at k_grid_mfma_wide). In the fixed scratch block, single
+    // precision with one output on multiples of 16 only: other tilings hold
+    // more buckets, and calls near the block's limit would no longer fit.
+    const int mu = mfma_tile(g.nu, g.supp), mv = mfma_tile(g.nv, g.supp);
+    const bool fits = fixed ? sizeof(T) == 4 && nout == 1 && g.nu % kMfmaTile == 0 && g.nv % kMfmaTile == 0
+                            : mu > 0 && mv > 0;
+    g.mfma = !degrid && g.wgrid && g.supp <= max_support<T>() && tile == 0 && fits && mfma_enabled() ? 1 : 0;
+    if (g.mfma) {
+        g.Tu = mu;
+        g.Tv = mv;
+    }
+    g.ntu = (g.nu + g.Tu - 1) / g.Tu;
+    g.ntv = (g.nv + g.Tv - 1) / g.Tv;
     const long long nkeys = (long long)g.ntu * g.ntv * 4 * g.nb;
     if (nkeys >= 0xffffffffll) {
         err = "grid too large for one call";
@@ -3653,6 +3820,7 @@ struct GridPrep {
     Tables<T> tb;
     LongTabs<T> lt;
     int P = 0, G_planes = 0, ngroups = 0, ntg = 0, TvP = 0;
+    std::uint32_t rc = kGridChunk;  // visibilities per item
     std::size_t lds = 0;
     std::uint32_t* item_off = nullptr;
     long long ub = 0;  // workgroups of the gridding launch
@@ -3675,8 +3843,8 @@ void grid_prepare(Workspace& ws, const Geometry& G, const Geo& g, const std::uin
     // padded row stride: TvP = S (mod 32) spreads a footprint's rows over the banks
     gp.TvP = g.Tv + ((g.supp - g.Tv) % 32 + 32) % 32;
     if (g.mfma) {
-        // the matrix cores hold kMfmaPlanes planes of a tile in registers
-        // (groups of 8 measured faster than balanced ones: 133 vs 139 ms)
+        // the matrix cores hold these planes of a tile in registers (groups
+        // of 8 measured faster than balanced ones: 133 vs 139 ms)
         gp.G_planes = std::max(1, std::min(P, kMfmaPlanes));
         gp.lds = 0;
     } else {
@@ -3686,6 +3854,7 @@ void grid_prepare(Workspace& ws, const Geometry& G, const Geo& g, const std::uin
         gp.G_planes = std::max(1, std::min({P, int(grid_lds<T>() / per_plane), 32}));
         gp.lds = per_plane * std::min(P, gp.G_planes);
     }
+    gp.rc = grid_chunk(g);
     gp.ngroups = (P + gp.G_planes - 1) / gp.G_planes;
     gp.ntg = g.ntu * g.ntv * gp.ngroups;
     const int ntg = gp.ntg;
@@ -3693,7 +3862,7 @@ void grid_prepare(Workspace& ws, const Geometry& G, const Geo& g, const std::uin
     gp.item_off = static_cast<std::uint32_t*>(ws.get(kSlotItemOff, sizeof(std::uint32_t) * (ntg + 1)));
     if (!cache || !cache->valid) {
         k_grid_items<<<(ntg + 1 + 255) / 256, 256, 0, st>>>(g, off, gp.tb.order, gp.G_planes, gp.ngroups, g.supp,
-                                                             kGridChunk, items);
+                                                             gp.rc, items);
         HIPCHK(hipGetLastError());
         exclusive_scan(ws, items, gp.item_off, ntg + 1, st);
     }
@@ -3801,13 +3970,12 @@ void grid_pipeline(Workspace& ws, const Geometry& G, const Geo& g, const DevIn& 
                    T* psf, hipStream_t st, HostKeep& keep, StageTimer& timer, ItemCache* cache = nullptr) {
     GridPrep<T> gp;
     grid_prepare<T>(ws, G, g, off, nout, st, keep, timer, cache, gp);
-    const std::uint32_t rc = kGridChunk;
+    const std::uint32_t rc = gp.rc;
     if (gp.ub == 0) {
         // nothing to grid: every cell was cleared above
     } else if (g.mfma) {
-        if constexpr (sizeof(T) == 4)
-            launch_grid_mfma(g.supp, int(gp.ub), form, st, g, recs, off, gp.tb.coeff, din, gp.G_planes, gp.ngroups,
-                             rc, gp.item_off, gp.tb.order, gp.grid);
+        launch_grid_mfma<T>(g.supp, int(gp.ub), nout, form, st, g, recs, off, gp.tb.coeff, din, gp.G_planes,
+                            gp.ngroups, rc, gp.item_off, gp.tb.order, gp.grid);
     } else if (nout == 2)
         launch_grid<T, 2, false>(g.supp, int(gp.ub), gp.lds, st, g, recs, off, gp.tb.coeff, din, gp.G_planes,
                                  gp.ngroups, gp.TvP, rc, gp.item_off, gp.tb.order, gp.grid);
@@ -3855,7 +4023,7 @@ int vis2dirty_on(bool fixed, const Options& o, const DevInputs& in, const double
         Geometry G;
         if (!make_geometry(o, sizeof(T) == 4, std::size_t(nvis), wlo, whi, G, err)) return 1;
         const int nout = (dirty ? 1 : 0) + (psf ? 1 : 0);
-        if (!fill_geo<T>(G, g, nout, false, err, tile)) return 1;
+        if (!fill_geo<T>(G, g, nout, false, err, tile, fixed)) return 1;
         Rec<T>* recs;
         std::uint32_t* off;
         if (use_vis)
@@ -4175,9 +4343,12 @@ int device_batch_vis2dirty(BatchImage* imgs, int n, std::size_t budget, hipStrea
             while (end < order.size() && (end == at || used + plans[order[end]].bytes <= budget))
                 used += plans[order[end++]].bytes;
             std::vector<GridPrep<T>> preps(end - at);
-            std::vector<GridJob<T>> jobs, mjobs;  // LDS gridding, matrix-core gridding
+            // LDS gridding; matrix-core gridding (in double precision by support)
+            std::vector<GridJob<T>> jobs;
+            std::map<int, std::vector<GridJob<T>>> mjobs;
             std::size_t lds = 0;
-            long long total = 0, mtotal = 0;
+            long long total = 0;
+            std::map<int, long long> mtotal;
             for (std::size_t k = at; k < end; ++k) {
                 const int i = order[k];
                 Plan& pl = plans[i];
@@ -4189,35 +4360,42 @@ int device_batch_vis2dirty(BatchImage* imgs, int n, std::size_t budget, hipStrea
                 GridPrep<T>& gp = preps[k - at];
                 grid_prepare<T>(ws, pl.G, pl.g, off, 1, st, keep, timer, nullptr, gp);
                 if (gp.ub == 0) continue;
-                long long& tot = pl.g.mfma ? mtotal : total;
+                const int kind = sizeof(T) == 4 ? 0 : pl.g.supp;
+                long long& tot = pl.g.mfma ? mtotal[kind] : total;
                 if (tot + gp.ub >= (1LL << 31)) throw DevError{"too many gridding items in one batch"};
-                (pl.g.mfma ? mjobs : jobs)
+                (pl.g.mfma ? mjobs[kind] : jobs)
                     .push_back(GridJob<T>{pl.g, recs, off, gp.tb.coeff, pl.din, gp.G_planes, gp.ngroups, gp.TvP,
-                                          kGridChunk, gp.item_off, gp.tb.order, gp.grid, std::uint32_t(tot)});
+                                          gp.rc, gp.item_off, gp.tb.order, gp.grid, std::uint32_t(tot)});
                 tot += gp.ub;
                 if (!pl.g.mfma) lds = std::max(lds, gp.lds);
             }
             timer.mark("sort");
             // the job tables to the device: one launch per gridding kernel
-            auto upload = [&](const std::vector<GridJob<T>>& js, int slot) {
+            std::size_t ntab = jobs.size();
+            for (const auto& m : mjobs) ntab += m.second.size();
+            GridJob<T>* dj = ntab ? static_cast<GridJob<T>*>(pool.control.get(kSlotItems, sizeof(GridJob<T>) * ntab)) : nullptr;
+            auto upload = [&](const std::vector<GridJob<T>>& js) {
                 keep.b.emplace_back(reinterpret_cast<const char*>(js.data()),
                                     reinterpret_cast<const char*>(js.data() + js.size()));
-                const std::size_t jb = sizeof(GridJob<T>) * js.size();
-                void* dj = pool.control.get(slot, jb);
-                HIPCHK(hipMemcpyAsync(dj, keep.b.back().data(), jb, hipMemcpyHostToDevice, st));
-                return static_cast<const GridJob<T>*>(dj);
+                GridJob<T>* at_ = dj;
+                HIPCHK(hipMemcpyAsync(at_, keep.b.back().data(), sizeof(GridJob<T>) * js.size(), hipMemcpyHostToDevice, st));
+                dj += js.size();
+                return static_cast<const GridJob<T>*>(at_);
             };
             if (!jobs.empty()) {
-                const GridJob<T>* dj = upload(jobs, kSlotItems);
+                const GridJob<T>* d = upload(jobs);
                 lds_limit((const void*)k_grid_jobs<T, 1, false>, lds);
-                k_grid_jobs<T, 1, false><<<int(total), grid_threads<T>(), lds, st>>>(dj, int(jobs.size()));
+                k_grid_jobs<T, 1, false><<<int(total), grid_threads<T>(), lds, st>>>(d, int(jobs.size()));
                 HIPCHK(hipGetLastError());
             }
-            if constexpr (sizeof(T) == 4) {
-                if (!mjobs.empty()) {
-                    const GridJob<T>* dj = upload(mjobs, kSlotItemOff);
-                    k_grid_mfma_jobs<false><<<int(mtotal), 64, 0, st>>>(dj, int(mjobs.size()));
+            for (const auto& m : mjobs) {
+                const GridJob<T>* d = upload(m.second);
+                const int njobs = int(m.second.size()), blocks = int(mtotal[m.first]);
+                if constexpr (sizeof(T) == 4) {
+                    k_grid_mfma_jobs<false><<<blocks, 64, 0, st>>>(d, njobs);
                     HIPCHK(hipGetLastError());
+                } else {
+                    launch_jobs64(m.first, blocks, st, d, njobs);
                 }
             }
             timer.mark("grid");

@@ -360,3 +360,49 @@ def test_cells_no_visibility_reaches_are_cleared(occ, monkeypatch):
         got, ref, info, _ = v2d(uvw, freq, vis, wgt, nx, ny, dx, eps, single, mask=keep)
         assert info["nvis"] == int(keep.sum())
         assert rel_linf(got, ref) < TOL_ORACLE[single]
+
+
+# the matrix-core gridding where its tiles end: grid sides of every residue
+# modulo the 16-cell window (whole, short, and last tiles below the support,
+# which shrink the tile), every support, one output and two
+@pytest.mark.parametrize("nu,nv", [(64, 66), (70, 72), (84, 90), (98, 60), (66, 100), (110, 54)])
+@pytest.mark.parametrize("single,supp", [(True, s) for s in range(4, 9)] + [(False, s) for s in range(4, 17)])
+def test_matrix_core_tiles_on_any_grid(nu, nv, single, supp):
+    rows = [k for k, r in enumerate(W.kernel_table()) if r[0] == supp and (r[6] or not single) and r[1] < 1.7]
+    kernel = (rows[len(rows) // 2], nu, nv)
+    uvw, freq, vis, wgt, nx, ny, dx = ref_case(nx=32, ny=30, field=0.3, wmax=900.0, nrow=90, seed=nu + supp)
+    uvw[:40, :2] *= 0.02  # a crowded tile: several items
+    got, ref, info, rinfo = v2d(uvw, freq, vis, wgt, nx, ny, dx, 1e-3, single, kernel=kernel)
+    same_plan(info, rinfo)
+    assert rel_linf(got, ref) < TOL_ORACLE[single]
+    cv = vis.astype(np.complex64 if single else np.complex128)
+    rw = wgt.astype(np.float32 if single else np.float64)
+    common = dict(npix_x=nx, npix_y=ny, pixsize_x=dx, pixsize_y=dx, epsilon=1e-3, kernel=kernel)
+    dirty, psf = W.dirty_psf(uvw=uvw, freq=freq, vis=cv, wgt=rw, single=single, **common)
+    both, _ = O.vis2dirty(uvw, freq, cv, rw, single=single, outputs=("dirty", "psf"), **common)
+    assert rel_linf(dirty, both["dirty"]) < TOL_ORACLE[single]
+    assert rel_linf(psf, both["psf"]) < TOL_ORACLE[single]
+
+
+def test_double_batch_on_the_matrix_cores():
+    # one launch per support, images of several supports in one batch
+    import torch
+    from rang import batch
+
+    made = []
+    for k, (eps, nx, ny) in enumerate([(1e-4, 40, 36), (1e-7, 32, 48), (1e-11, 48, 32), (1e-7, 60, 40)]):
+        uvw, freq, vis, wgt, _, _, _ = ref_case(nx=nx, ny=ny, field=0.3, wmax=700.0, nrow=60, seed=30 + k)
+        dx = 0.3 / nx
+        opts = [nx, ny, dx, dx, eps, 0, 0, 1.1, 2.6, 1, 0, 0, 0, 0, 1, -1, 0, 0]
+        im = batch.Image(opts, torch.from_numpy(uvw).cuda(), freq, torch.from_numpy(vis).cuda(),
+                         torch.from_numpy(wgt).cuda())
+        ref, rinfo = O.vis2dirty(uvw, freq, vis, wgt, npix_x=nx, npix_y=ny, pixsize_x=dx, pixsize_y=dx, epsilon=eps,
+                                 single=False)
+        made.append((im, ref["dirty"], rinfo))
+    out = batch.vis2dirty([m[0] for m in made], single=False)
+    assert len({int(m[0].info[1]) for m in made}) >= 3
+    for (im, ref, rinfo), d in zip(made, out):
+        assert [int(v) for v in im.info[:6]] == [int(v) for v in rinfo[:6]]
+        # support 13 at oversampling 1.35: the correction at the image's edge
+        # amplifies the sums' rounding by 1e5 (5e-11 with the LDS gridder too)
+        assert rel_linf(d.cpu().numpy(), ref) < 1e-10
