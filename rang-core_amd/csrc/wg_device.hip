@@ -3,8 +3,9 @@
 // vis2dirty (rang-core core/src/wgridder.rs:2436-2683):
 //   scan      active count and |w| range                    (k_scan)
 //   plan      kernel, grid and w-planes on the host, FP64    (wg_plan.cpp)
-//   sort      bucket key per visibility, counts, prefix sum, (k_keys, scan,
-//             one record per active visibility in bucket order  k_scatter)
+//   sort      rank in its bucket per visibility, counts,    (k_ranks, scan,
+//             prefix sum, one record per active visibility    k_scatter)
+//             in bucket order
 //   grid      one workgroup per (uv tile, group of w-planes, chunk of up to
 //             4096 visibilities) gathers the visibilities of its tile and of
 //             the three tiles whose footprints reach into it, accumulates in
@@ -129,7 +130,6 @@ enum Slot : int {
     kSlotKeys,
     kSlotCounts,
     kSlotOffsets,
-    kSlotCursor,
     kSlotScan,
     kSlotRecs,
     kSlotCoeff,
@@ -152,7 +152,6 @@ enum Slot : int {
     kSlotKeys2,
     kSlotCounts2,
     kSlotOffsets2,
-    kSlotCursor2,
     kSlotRecs2,
     kSlotOrder2,
     // prepared calls: visibility buffer, reductions, solver vectors
@@ -358,6 +357,8 @@ struct Geo {
     int shifting, lmshift;
     double fu, fv, fw;
     int Tu, Tv, ntu, ntv;
+    unsigned mTu, mTv;  // tile_of's multipliers of the tile sides
+    double inv_nchan;
     int tnx, tny;
     int divide_by_n;
     // Image-side arrays column-major (index j nx + i): the w-screen and
@@ -473,21 +474,39 @@ __device__ __forceinline__ bool active(const DevIn& in, long long i) {
     return tnorm * twgt * tmask != 0.0;
 }
 
+// The first cell of a footprint and the position from it. u + ushift lies in
+// [nu - supp / 2, 2 nu + 1): 32-bit cells, one conditional step to wrap them.
 __device__ __forceinline__ void getpix(const Geo& g, double uin, double vin, double& uf,
-                                       double& vf, long long& iu0, long long& iv0) {
+                                       double& vf, int& iu0, int& iv0) {
     double u = uin * g.pixsize_x;
     u = (u - floor(u)) * double(g.nu);
-    iu0 = min((long long)(u + g.ushift) - g.nu, g.maxiu0);
+    iu0 = min(int(u + g.ushift) - g.nu, int(g.maxiu0));
     uf = u - double(iu0);
     double v = vin * g.pixsize_y;
     v = (v - floor(v)) * double(g.nv);
-    iv0 = min((long long)(v + g.vshift) - g.nv, g.maxiv0);
+    iv0 = min(int(v + g.vshift) - g.nv, int(g.maxiv0));
     vf = v - double(iv0);
 }
 
-__device__ __forceinline__ int shifted(long long i0, int n) {
-    long long v = (i0 + n / 2) % n;
-    return int(v < 0 ? v + n : v);
+// (i0 + n / 2) mod n for i0 in [-n / 2, n + n / 2).
+__device__ __forceinline__ int shifted(int i0, int n) {
+    int v = i0 + n / 2;
+    if (v < 0) v += n;
+    return v >= n ? v - n : v;
+}
+
+// x / d with m = ceil(2^32 / d): exact for x d < 2^32 (grid sides below 2^20
+// times tiles of 8 to 64 cells).
+__device__ __forceinline__ int tile_of(int x, unsigned m) { return int(__umulhi(unsigned(x), m)); }
+
+// Row of sample i: the product with 1 / nchan is off by less than one unit in
+// the last place of a double, so its floor by at most one.
+__device__ __forceinline__ unsigned row_of(const Geo& g, unsigned i) {
+    unsigned r = unsigned(double(i) * g.inv_nchan);
+    const unsigned nchan = unsigned(g.nchan);
+    if (r * nchan > i) --r;
+    if (i - r * nchan >= nchan) ++r;
+    return r;
 }
 
 __device__ __forceinline__ int minplane(const Geo& g, double w) {
@@ -529,7 +548,7 @@ __global__ __launch_bounds__(256) void k_scan(DevIn in, Geo g, unsigned long lon
     const unsigned stride = gridDim.x * blockDim.x;
     for (unsigned i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) {
         if (!active<T, USE_VIS>(in, i)) continue;
-        const unsigned row = i / nchan, ch = i - row * nchan;
+        const unsigned row = row_of(g, i), ch = i - row * nchan;
         const double w = fabs(g.fw * in.uvw[3 * row + 2] * in.foc[ch]);
         ++cnt;
         lo = fmin(lo, w);
@@ -589,26 +608,38 @@ __global__ __launch_bounds__(256) void k_scan_final(const unsigned long long* bc
 
 // ------------------------------------------------------------ sort
 
-// Bucket of an active visibility: (tile, spill class, first plane). The
-// spill class says whether its footprint reaches the next tile in u (2) and
-// in v (1).
-template <class T, bool USE_VIS>
-__device__ __forceinline__ std::uint32_t key_of(const DevIn& in, const Geo& g, unsigned i,
-                                                unsigned row, unsigned ch) {
-    if (!active<T, USE_VIS>(in, i)) return kNoKey;
+// Where a visibility falls on the grid: its FixW-signed coordinates, the
+// position of its footprint and its bucket (tile, spill class, first plane).
+// The spill class says whether its footprint reaches the next tile in u (2)
+// and in v (1).
+struct Place {
+    double imflip, b[3];  // the sign of w and the coordinates times it
+    double w, uf, vf;
+    int ou, ov, mp;
+    std::uint32_t key;
+};
+
+__device__ __forceinline__ Place place_of(const DevIn& in, const Geo& g, unsigned row, unsigned ch) {
+    Place r;
     double c[3];
     coord_of(in, g, int(row), c);
-    const double sgn = c[2] < 0.0 ? -1.0 : 1.0;
+    r.imflip = c[2] < 0.0 ? -1.0 : 1.0;  // FixW (wgridder.rs:583-586)
+    r.b[0] = c[0] * r.imflip;
+    r.b[1] = c[1] * r.imflip;
+    r.b[2] = c[2] * r.imflip;
     const double f = in.foc[ch];
-    const double u = c[0] * sgn * f, v = c[1] * sgn * f, w = c[2] * sgn * f;
-    double uf, vf;
-    long long iu0, iv0;
-    getpix(g, u, v, uf, vf, iu0, iv0);
+    const double u = r.b[0] * f, v = r.b[1] * f;
+    r.w = r.b[2] * f;
+    int iu0, iv0;
+    getpix(g, u, v, r.uf, r.vf, iu0, iv0);
     const int su = shifted(iu0, g.nu), sv = shifted(iv0, g.nv);
-    const int tu = su / g.Tu, tv = sv / g.Tv;
-    const int ou = su - tu * g.Tu, ov = sv - tv * g.Tv;
-    const int cat = ((ou + g.supp > tile_wu(g, tu)) ? 2 : 0) | ((ov + g.supp > tile_wv(g, tv)) ? 1 : 0);
-    return std::uint32_t((((long long)tu * g.ntv + tv) * 4 + cat) * g.nb + minplane(g, w));
+    const int tu = tile_of(su, g.mTu), tv = tile_of(sv, g.mTv);
+    r.ou = su - tu * g.Tu;
+    r.ov = sv - tv * g.Tv;
+    const int cat = ((r.ou + g.supp > tile_wu(g, tu)) ? 2 : 0) | ((r.ov + g.supp > tile_wv(g, tv)) ? 1 : 0);
+    r.mp = minplane(g, r.w);
+    r.key = std::uint32_t((((long long)tu * g.ntv + tv) * 4 + cat) * g.nb + r.mp);
+    return r;
 }
 
 // Runs of equal keys among the consecutive lanes of a wave (channels of one
@@ -627,24 +658,31 @@ __device__ __forceinline__ void wave_runs(std::uint32_t key, bool& head, int& le
     len = (after ? __ffsll((long long)after) - 1 : 64) - lane;
 }
 
-// One thread per visibility (coalesced); the first lane of each run adds the
-// run's length to its bucket's count.
+// Each active visibility's rank in its bucket (kNoKey for the others) and the
+// buckets' counts, one thread per visibility (coalesced): the first lane of
+// each run adds the run's length to its bucket's count, and what the count
+// was before gives the ranks. The scatter then needs no atomics of its own:
+// the random atomics of sparsely filled buckets bound the sort (116 M
+// visibilities over 88 M buckets: keys and scatter with an atomic each 4.4 +
+// 6.6 ms, ranks and scatter 4.5 + 4.3 ms; 3.2 M visibilities 107 + 130 -> 110
+// + 61 us; the index arithmetic does not show in either).
 template <class T, bool USE_VIS>
-__global__ __launch_bounds__(256) void k_keys(DevIn in, Geo g, std::uint32_t* keys,
-                                              std::uint32_t* counts) {
-    const unsigned n = unsigned(g.n), nchan = unsigned(g.nchan);
+__global__ __launch_bounds__(256) void k_ranks(DevIn in, Geo g, std::uint32_t* __restrict__ ranks,
+                                               std::uint32_t* __restrict__ counts) {
+    const unsigned n = unsigned(g.n);
     const unsigned i = blockIdx.x * blockDim.x + threadIdx.x;
-    const bool inside = i < n;
     std::uint32_t key = kNoKey;
-    if (inside) {
-        const unsigned row = i / nchan;
-        key = key_of<T, USE_VIS>(in, g, i, row, i - row * nchan);
-        keys[i] = key;
+    if (i < n && active<T, USE_VIS>(in, i)) {
+        const unsigned row = row_of(g, i);
+        key = place_of(in, g, row, i - row * unsigned(g.nchan)).key;
     }
     bool head;
     int len, pos, headlane;
     wave_runs(key, head, len, pos, headlane);
-    if (head && key != kNoKey) atomicAdd(&counts[key], std::uint32_t(len));
+    std::uint32_t base = 0;
+    if (head && key != kNoKey) base = atomicAdd(&counts[key], std::uint32_t(len));
+    base = __shfl(base, headlane, 64);
+    if (i < n) ranks[i] = key == kNoKey ? kNoKey : base + std::uint32_t(pos);
 }
 
 constexpr int kScanItems = 4096;  // per block of 1024 threads
@@ -685,25 +723,16 @@ __global__ __launch_bounds__(256) void k_scan_add(std::uint32_t* out, const std:
 // One record per active visibility in bucket order. MODE 0: a dirty image
 // alone (the data value), 1: with a PSF (the unit value; the data value is
 // formed while gridding), 2: dirty2vis (weight times conjugate shift phase).
-// One thread per row; each run of channels in one bucket takes a contiguous
-// block of slots with one atomic, in channel order.
 template <class T, int MODE>
-__device__ __forceinline__ Rec<T> make_rec(const DevIn& in, const Geo& g, unsigned i, int ch,
-                                           const double c[3], std::uint32_t key) {
-    const double imflip = c[2] < 0.0 ? -1.0 : 1.0;  // FixW (wgridder.rs:583-586)
-    const double b[3] = {c[0] * imflip, c[1] * imflip, c[2] * imflip};
+__device__ __forceinline__ Rec<T> make_rec(const DevIn& in, const Geo& g, unsigned i, int ch, const Place& at) {
+    const double imflip = at.imflip;
+    const double(&b)[3] = at.b;
     const double f = in.foc[ch];
-    const double u = b[0] * f, v = b[1] * f, w = b[2] * f;
-    double uf, vf;
-    long long iu0, iv0;
-    getpix(g, u, v, uf, vf, iu0, iv0);
-    const int su = shifted(iu0, g.nu), sv = shifted(iv0, g.nv);
-    const int ou = su % g.Tu, ov = sv % g.Tv;
     Rec<T> r;
-    r.w = w;
-    r.x0 = T(-uf * 2.0 + (double(g.supp) - 1.0));
-    r.y0 = T(-vf * 2.0 + (double(g.supp) - 1.0));
-    r.pos = std::uint32_t(ou) | (std::uint32_t(ov) << 8) | (std::uint32_t(key % std::uint32_t(g.nb)) << 16);
+    r.w = at.w;
+    r.x0 = T(-at.uf * 2.0 + (double(g.supp) - 1.0));
+    r.y0 = T(-at.vf * 2.0 + (double(g.supp) - 1.0));
+    r.pos = std::uint32_t(at.ou) | (std::uint32_t(at.ov) << 8) | (std::uint32_t(at.mp) << 16);
     r.idx = i | (imflip < 0.0 ? kFlip : 0u);
     T wv = T(1);
     const bool haswgt = wgt_get<T>(in, i, wv);
@@ -735,23 +764,15 @@ __device__ __forceinline__ Rec<T> make_rec(const DevIn& in, const Geo& g, unsign
 }
 
 template <class T, int MODE>
-__global__ __launch_bounds__(256) void k_scatter(DevIn in, Geo g, const std::uint32_t* keys,
-                                                 const std::uint32_t* offsets,
-                                                 std::uint32_t* cursor, Rec<T>* recs) {
-    const unsigned n = unsigned(g.n), nchan = unsigned(g.nchan);
+__global__ __launch_bounds__(256) void k_scatter(DevIn in, Geo g, const std::uint32_t* __restrict__ ranks,
+                                                 const std::uint32_t* __restrict__ offsets,
+                                                 Rec<T>* __restrict__ recs) {
     const unsigned i = blockIdx.x * blockDim.x + threadIdx.x;
-    const std::uint32_t key = i < n ? keys[i] : kNoKey;
-    bool head;
-    int len, pos, headlane;
-    wave_runs(key, head, len, pos, headlane);
-    std::uint32_t base = 0;
-    if (head && key != kNoKey) base = offsets[key] + atomicAdd(&cursor[key], std::uint32_t(len));
-    base = __shfl(base, headlane, 64);
-    if (key == kNoKey) return;
-    const unsigned row = i / nchan, ch = i - row * nchan;
-    double c[3];
-    coord_of(in, g, int(row), c);
-    recs[base + pos] = make_rec<T, MODE>(in, g, i, int(ch), c, key);
+    const std::uint32_t rank = i < unsigned(g.n) ? ranks[i] : kNoKey;
+    if (rank == kNoKey) return;
+    const unsigned row = row_of(g, i), ch = i - row * unsigned(g.nchan);
+    const Place at = place_of(in, g, row, ch);
+    recs[offsets[at.key] + rank] = make_rec<T, MODE>(in, g, i, int(ch), at);
 }
 
 // ------------------------------------------------------------ kernel taps
@@ -3294,6 +3315,8 @@ bool fill_geo(const Geometry& G, Geo& g, int nout, bool degrid, std::string& err
     }
     g.ntu = (g.nu + g.Tu - 1) / g.Tu;
     g.ntv = (g.nv + g.Tv - 1) / g.Tv;
+    g.mTu = fft_magic(unsigned(g.Tu));
+    g.mTv = fft_magic(unsigned(g.Tv));
     const long long nkeys = (long long)g.ntu * g.ntv * 4 * g.nb;
     if (nkeys >= 0xffffffffll) {
         err = "grid too large for one call";
@@ -3321,18 +3344,16 @@ void sort_records(Workspace& ws, const DevIn& din, const Geo& g, long long nvis,
                   Rec<T>** recs_out, std::uint32_t** off_out, int set = 0,
                   const DevIn* vals = nullptr) {
     const long long nkeys = (long long)g.ntu * g.ntv * 4 * g.nb;
-    std::uint32_t* keys = static_cast<std::uint32_t*>(ws.get(set ? kSlotKeys2 : kSlotKeys, sizeof(std::uint32_t) * g.n));
+    std::uint32_t* ranks = static_cast<std::uint32_t*>(ws.get(set ? kSlotKeys2 : kSlotKeys, sizeof(std::uint32_t) * g.n));
     std::uint32_t* counts = static_cast<std::uint32_t*>(ws.get(set ? kSlotCounts2 : kSlotCounts, sizeof(std::uint32_t) * (nkeys + 1)));
     std::uint32_t* off = static_cast<std::uint32_t*>(ws.get(set ? kSlotOffsets2 : kSlotOffsets, sizeof(std::uint32_t) * (nkeys + 1)));
-    std::uint32_t* cursor = static_cast<std::uint32_t*>(ws.get(set ? kSlotCursor2 : kSlotCursor, sizeof(std::uint32_t) * (nkeys + 1)));
     Rec<T>* recs = static_cast<Rec<T>*>(ws.get(set ? kSlotRecs2 : kSlotRecs, sizeof(Rec<T>) * std::max<long long>(nvis, 1)));
     fill_zero(counts, sizeof(std::uint32_t) * (nkeys + 1), st);
-    fill_zero(cursor, sizeof(std::uint32_t) * (nkeys + 1), st);
     const int eblocks = int((g.n + 255) / 256);
-    k_keys<T, USE_VIS><<<eblocks, 256, 0, st>>>(din, g, keys, counts);
+    k_ranks<T, USE_VIS><<<eblocks, 256, 0, st>>>(din, g, ranks, counts);
     HIPCHK(hipGetLastError());
     exclusive_scan(ws, counts, off, nkeys + 1, st);
-    k_scatter<T, MODE><<<eblocks, 256, 0, st>>>(vals ? *vals : din, g, keys, off, cursor, recs);
+    k_scatter<T, MODE><<<eblocks, 256, 0, st>>>(vals ? *vals : din, g, ranks, off, recs);
     HIPCHK(hipGetLastError());
     *recs_out = recs;
     *off_out = off;
@@ -3343,6 +3364,7 @@ Geo base_geo(std::size_t nrow, std::size_t nchan, const Options& o) {
     g.n = (long long)(nrow * nchan);
     g.nrow = int(nrow);
     g.nchan = int(nchan);
+    g.inv_nchan = nchan ? 1.0 / double(nchan) : 0.0;
     double r_l, r_m;
     recentring(o, r_l, r_m);
     g.r_l = r_l;
@@ -4894,9 +4916,8 @@ PreparedBase* prepared_new(const Options& o, const DevInputs& in, const double* 
             HIPCHK(hipGetLastError());
         }
         HIPCHK(hipStreamSynchronize(st));
-        // the sort's per-visibility keys, counts and cursors are not needed again
-        for (int k : {int(kSlotKeys), int(kSlotKeys2), int(kSlotCounts), int(kSlotCounts2), int(kSlotCursor),
-                      int(kSlotCursor2)}) {
+        // the sort's per-visibility ranks and its counts are not needed again
+        for (int k : {int(kSlotKeys), int(kSlotKeys2), int(kSlotCounts), int(kSlotCounts2)}) {
             if (p->ws.ptr[k]) HIPCHK(hipFree(p->ws.ptr[k]));
             p->ws.ptr[k] = nullptr;
             p->ws.size[k] = 0;
