@@ -2638,6 +2638,34 @@ struct DegridOut {
     double* part = nullptr;
 };
 
+// The value of record r from its sum over the grid: the weight and shift phase,
+// and where it goes (DegridOut).
+template <class T>
+__device__ __forceinline__ void degrid_store(const Geo& g, const Rec<T>& rec, std::uint32_t r, cx<T> out,
+                                             const DegridOut<T>& o, double& mis) {
+    cx<T> res;
+    if (g.shifting)
+        res = cmul(out, cx<T>{rec.re, rec.im});
+    else
+        res = {out.re * rec.re, out.im * rec.re};
+    const std::uint32_t idx = rec.idx & ~kFlip;
+    if (o.mode == 0) {
+        o.vis[idx] = res;
+        return;
+    }
+    const std::uint32_t k0 = o.pos[r];
+    if (o.mode == 1) {
+        o.stored[k0] = res;
+        return;
+    }
+    const cx<T> d = vis_get<T>(o.data, o.sorted ? (long long)k0 : (long long)idx);
+    const cx<T> q = {d.re - res.re, d.im - res.im};
+    o.stored[k0] = q;
+    T wv = T(1);
+    wgt_get<T>(o.data, idx, wv);
+    mis += double(wv) * (double(q.re) * double(q.re) + double(q.im) * double(q.im));
+}
+
 template <class T, int S, bool STAGE>
 __global__ __launch_bounds__((degrid_threads<T, STAGE>())) void k_degrid(Geo g, const Rec<T>* __restrict__ recs,
                                                 const std::uint32_t* __restrict__ off,
@@ -2758,27 +2786,7 @@ __global__ __launch_bounds__((degrid_threads<T, STAGE>())) void k_degrid(Geo g, 
             }
             out = {rr + out.re, ri * fl + out.im};
         }
-        cx<T> res;
-        if (g.shifting)
-            res = cmul(out, cx<T>{rc_.re, rc_.im});
-        else
-            res = {out.re * rc_.re, out.im * rc_.re};
-        const std::uint32_t idx = rc_.idx & ~kFlip;
-        if (o.mode == 0) {
-            o.vis[idx] = res;
-        } else {
-            const std::uint32_t k0 = o.pos[r];
-            if (o.mode == 1) {
-                o.stored[k0] = res;
-            } else {
-                const cx<T> d = vis_get<T>(o.data, o.sorted ? (long long)k0 : (long long)idx);
-                const cx<T> q = {d.re - res.re, d.im - res.im};
-                o.stored[k0] = q;
-                T wv = T(1);
-                wgt_get<T>(o.data, idx, wv);
-                mis += double(wv) * (double(q.re) * double(q.re) + double(q.im) * double(q.im));
-            }
-        }
+        degrid_store(g, rc_, r, out, o, mis);
     }
     if (o.mode == 2) {
         // the workgroup's misfit: lanes, then waves
@@ -2792,6 +2800,138 @@ __global__ __launch_bounds__((degrid_threads<T, STAGE>())) void k_degrid(Geo g, 
             for (int k = 0; k < int(blockDim.x) / 64; ++k) t += wsum[k];
             o.part[blockIdx.x] = t;
         }
+    }
+}
+
+// d2v in double precision on the matrix cores: one wave per item, 16
+// visibilities of one tile at a time. Their sums over the 32 x 32 cells from
+// the tile's first one (which hold every footprint that starts in a tile of at
+// most 16) go block by block of 16 x 16 cells and plane by plane:
+// Y[i][k] = sum_j G[i][j] kv_k(j - ov_k), four v_mfma_f64_16x16x4_f64 per part
+// with the plane's cells as the first operand, read from memory in the
+// operand's layout, and then sum_i ku_k(i - ou_k) Y[i][k] kw_k on the vector
+// unit. Blocks that no footprint of the sixteen reaches, and planes outside
+// the union of theirs, are skipped (records come sorted by spill class and
+// first plane). A visibility per thread reading its S^3 cells from memory left
+// a call of 118 k visibilities at support 11 with 1.8 waves per SIMD (706 us,
+// this kernel 184 us).
+template <int S>
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 4))) void k_degrid_mfma(
+    Geo g, const Rec<double>* __restrict__ recs, const std::uint32_t* __restrict__ off,
+    const double* __restrict__ coeff, const cx<double>* __restrict__ grid, std::uint32_t rc,
+    const std::uint32_t* __restrict__ item_off, const std::uint32_t* __restrict__ order, DegridOut<double> o) {
+    constexpr int NE = ne_of<S>();
+    __shared__ double coef[2 * NE * S];
+    __shared__ double s_tap[3][16][17];
+    const int lane = threadIdx.x, k = lane & 15, q = lane >> 4;
+    int rank;
+    std::uint32_t chunk, nchunks;
+    if (!find_item(item_off, g.ntu * g.ntv, blockIdx.x, rank, chunk, nchunks)) return;
+    const int tile = int(order[rank]);
+    const std::uint32_t t0 = off[(long long)tile * 4 * g.nb], t1 = off[(long long)(tile + 1) * 4 * g.nb];
+    const std::uint32_t a = t0 + chunk * rc, b = min(t1, a + rc);
+    for (int e = lane; e < 2 * NE * S; e += 64) coef[e] = coeff[e];
+    const int tu = tile / g.ntv, tv = tile - tu * g.ntv;
+    const long long plane = (long long)g.nu * g.nv;
+    // this lane's cells of the first operand: row k of each block row, columns
+    // 4 s + q of each block column. Rows past the tile's halo are not read:
+    // the row transform may have left them unwritten
+    long long row[2];
+    int col[2][4];
+    bool live[2];
+#pragma unroll
+    for (int bl = 0; bl < 2; ++bl) {
+        live[bl] = 16 * bl + k < g.Tu + S - 1;
+        row[bl] = (long long)((tu * g.Tu + 16 * bl + k + g.nu / 2) % g.nu) * g.nv;
+#pragma unroll
+        for (int s = 0; s < 4; ++s) col[bl][s] = vpos(g, (tv * g.Tv + 16 * bl + 4 * s + q + g.nv / 2) % g.nv);
+    }
+    double mis = 0.0;
+    for (std::uint32_t r0 = a; r0 < b; r0 += 16) {
+        const bool on = r0 + k < b;
+        Rec<double> rec{};
+        if (on) rec = recs[r0 + k];
+        const int ou = int(rec.pos & 255u), ov = int((rec.pos >> 8) & 255u), mp = int(rec.pos >> 16);
+        __syncthreads();  // the previous taps are consumed
+#pragma unroll
+        for (int t4 = 0; t4 < S; t4 += 4) {
+            const int t = t4 + q;
+            if (t < S) {
+                s_tap[0][k][t] = eval_tap<double, S>(coef, t, rec.x0);
+                s_tap[1][k][t] = eval_tap<double, S>(coef, t, rec.y0);
+                s_tap[2][k][t] = w_factor<double, S>(g, coef, t, mp + t, rec.w);
+            }
+        }
+        __syncthreads();
+        // ku at the result rows q + 4 r, kv at the operand rows 4 s + q
+        double ku[2][4], kv[2][4];
+#pragma unroll
+        for (int bl = 0; bl < 2; ++bl)
+#pragma unroll
+            for (int s = 0; s < 4; ++s) {
+                const int tu_ = 16 * bl + q + 4 * s - ou, tv_ = 16 * bl + 4 * s + q - ov;
+                ku[bl][s] = on && tu_ >= 0 && tu_ < S ? s_tap[0][k][tu_] : 0.0;
+                kv[bl][s] = on && tv_ >= 0 && tv_ < S ? s_tap[1][k][tv_] : 0.0;
+            }
+        // the union of the sixteen's planes, and the blocks they reach
+        int plo = on ? mp : g.nplanes, phi = on ? mp + S : 0;
+#pragma unroll
+        for (int h = 1; h < 16; h <<= 1) {
+            plo = min(plo, __shfl_xor(plo, h, 64));
+            phi = max(phi, __shfl_xor(phi, h, 64));
+        }
+        plo = __builtin_amdgcn_readfirstlane(plo);
+        phi = min(__builtin_amdgcn_readfirstlane(phi), g.nplanes);
+        const bool u1 = __any(on && ou + S > 16), v1 = __any(on && ov + S > 16);
+        const bool u0 = __any(on && ou < 16), v0 = __any(on && ov < 16);
+        double re = 0.0, im = 0.0;
+#pragma unroll
+        for (int bu = 0; bu < 2; ++bu)
+#pragma unroll
+            for (int bv = 0; bv < 2; ++bv) {
+                if (!(bu ? u1 : u0) || !(bv ? v1 : v0)) continue;
+                const cx<double>* src = grid + row[bu];
+                typedef double d2 __attribute__((ext_vector_type(2)));
+                d2 c[4], nx[4];
+#pragma unroll
+                for (int s = 0; s < 4; ++s)
+                    c[s] = live[bu] ? *reinterpret_cast<const d2*>(src + plo * plane + col[bv][s]) : d2{0.0, 0.0};
+                for (int p = plo; p < phi; ++p) {
+                    // the next plane's cells while this one's are multiplied
+                    const int pn = min(p + 1, phi - 1);
+#pragma unroll
+                    for (int s = 0; s < 4; ++s)
+                        nx[s] = live[bu] ? *reinterpret_cast<const d2*>(src + pn * plane + col[bv][s]) : d2{0.0, 0.0};
+                    const int t = p - mp;
+                    const double kw = t >= 0 && t < S ? s_tap[2][k][t] : 0.0;
+                    mfma_d4 yr{0.0, 0.0, 0.0, 0.0}, yi{0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+                    for (int s = 0; s < 4; ++s) {
+                        yr = Mfma<double>::mul(c[s].x, kv[bv][s], yr);
+                        yi = Mfma<double>::mul(c[s].y, kv[bv][s], yi);
+                    }
+                    double sr = 0.0, si = 0.0;
+#pragma unroll
+                    for (int s = 0; s < 4; ++s) {
+                        sr = fma(ku[bu][s], yr[s], sr);
+                        si = fma(ku[bu][s], yi[s], si);
+                        c[s] = nx[s];
+                    }
+                    re = fma(kw, sr, re);
+                    im = fma(kw, si, im);
+                }
+            }
+        // rows q + 4 r of the four lane groups
+        re += __shfl_xor(re, 16, 64);
+        im += __shfl_xor(im, 16, 64);
+        re += __shfl_xor(re, 32, 64);
+        im += __shfl_xor(im, 32, 64);
+        if (on && q == 0)
+            degrid_store(g, rec, r0 + k, cx<double>{re, (rec.idx & kFlip) ? -im : im}, o, mis);
+    }
+    if (o.mode == 2) {
+        for (int h = 32; h > 0; h >>= 1) mis += __shfl_down(mis, h, 64);
+        if (lane == 0) o.part[blockIdx.x] = mis;
     }
 }
 
@@ -2900,6 +3040,23 @@ void launch_degrid(int S, int nblocks, std::size_t lds, hipStream_t st, const Ge
         throw DevError{"unsupported kernel support"};
     }
 #undef DEGRID_CASE
+    HIPCHK(hipGetLastError());
+}
+
+void launch_degrid_mfma(int S, int nblocks, hipStream_t st, const Geo& g, const Rec<double>* recs,
+                        const std::uint32_t* off, const double* coeff, const cx<double>* grid, std::uint32_t rc,
+                        const std::uint32_t* item_off, const std::uint32_t* order, const DegridOut<double>& o) {
+#define DMFMA_CASE(SS)                                                                                 \
+    case SS:                                                                                           \
+        k_degrid_mfma<SS><<<nblocks, 64, 0, st>>>(g, recs, off, coeff, grid, rc, item_off, order, o); \
+        break;
+    switch (S) {
+        DMFMA_CASE(4) DMFMA_CASE(5) DMFMA_CASE(6) DMFMA_CASE(7) DMFMA_CASE(8) DMFMA_CASE(9) DMFMA_CASE(10)
+        DMFMA_CASE(11) DMFMA_CASE(12) DMFMA_CASE(13) DMFMA_CASE(14) DMFMA_CASE(15) DMFMA_CASE(16)
+    default:
+        throw DevError{"unsupported kernel support"};
+    }
+#undef DMFMA_CASE
     HIPCHK(hipGetLastError());
 }
 
@@ -3162,6 +3319,13 @@ constexpr std::size_t degrid_lds_max() {
     return sizeof(T) == 4 ? 150 * 1024 : 64 * 1024;
 }
 
+// Visibilities per item of the matrix-core degridding, one wave's serial work:
+// about 8192 items over the call, in whole groups of 16.
+std::uint32_t degrid_chunk_mfma(const Geo& g) {
+    const long long per = (g.n / 8192 + 15) / 16 * 16;
+    return std::uint32_t(std::max<long long>(32, std::min<long long>(1024, per)));
+}
+
 // Items per degridding launch and their records reordered within each item
 // (k_sort_chunks), before the degridder first reads them: the chunk size the
 // degrid pipeline will use for this geometry. RANG_DEGRID_SORT=0 leaves the
@@ -3173,6 +3337,8 @@ void sort_degrid_chunks(Workspace& ws, const Geo& g, Rec<T>* recs, const std::ui
         return !(e && e[0] == '0');
     }();
     if (!on) return;
+    // the matrix cores take the records as bucketed, by spill class and plane
+    if (g.mfma) return;
     const int P = g.wgrid ? g.nplanes : 1;
     const bool staged = degrid_lds<T>(g.Tu, g.Tv, g.supp, P) <= degrid_lds_max<T>();
     const std::uint32_t rc = staged ? degrid_chunk_staged<T>() : kDegridChunk;
@@ -3308,7 +3474,12 @@ bool fill_geo(const Geometry& G, Geo& g, int nout, bool degrid, std::string& err
     const int mu = mfma_tile(g.nu, g.supp), mv = mfma_tile(g.nv, g.supp);
     const bool fits = fixed ? sizeof(T) == 4 && nout == 1 && g.nu % kMfmaTile == 0 && g.nv % kMfmaTile == 0
                             : mu > 0 && mv > 0;
-    g.mfma = !degrid && g.wgrid && g.supp <= max_support<T>() && tile == 0 && fits && mfma_enabled() ? 1 : 0;
+    // degridding goes there in double precision where a tile's planes do not
+    // fit the staged LDS form (3.2 M visibilities at 1024^2, support 11: 11.6
+    // -> 4.8 ms; support 7, which fits, 1.7 ms staged and 3.0 ms there); in
+    // single precision the staged form is the faster one throughout
+    const bool unstaged = sizeof(T) == 8 && degrid_lds<T>(g.Tu, g.Tv, g.supp, P) > degrid_lds_max<T>();
+    g.mfma = (!degrid || unstaged) && g.wgrid && g.supp <= max_support<T>() && tile == 0 && fits && mfma_enabled() ? 1 : 0;
     if (g.mfma) {
         g.Tu = mu;
         g.Tv = mv;
@@ -4471,8 +4642,8 @@ void degrid_pipeline(Workspace& ws, const Geometry& G, const Geo& g, const Rec<T
     std::uint32_t* item_off = static_cast<std::uint32_t*>(
         ws.get(cache ? kSlotItemOff2 : kSlotItemOff, sizeof(std::uint32_t) * (nt + 1)));
     const std::size_t dl = degrid_lds<T>(g.Tu, g.Tv, g.supp, P);
-    const bool staged = dl <= degrid_lds_max<T>();
-    const std::uint32_t rc = staged ? degrid_chunk_staged<T>() : kDegridChunk;
+    const bool staged = !g.mfma && dl <= degrid_lds_max<T>();
+    const std::uint32_t rc = g.mfma ? degrid_chunk_mfma(g) : staged ? degrid_chunk_staged<T>() : kDegridChunk;
     long long ub;
     if (cache && cache->valid) {
         ub = cache->ub;
@@ -4547,6 +4718,9 @@ void degrid_pipeline(Workspace& ws, const Geometry& G, const Geo& g, const Rec<T
     if (o.mode == 2) o.part = static_cast<double*>(ws.get(kSlotRed, sizeof(double) * std::max<long long>(ub, 1)));
     if (ub == 0) {
         // nothing to degrid
+    } else if (g.mfma) {
+        if constexpr (sizeof(T) == 8)
+            launch_degrid_mfma(g.supp, int(ub), st, g, recs, off, tb.coeff, grid, rc, item_off, tb.order, o);
     } else if (staged)
         launch_degrid<T, true>(g.supp, int(ub), dl, st, g, recs, off, tb.coeff, grid, rc,
                                item_off, tb.order, o);

@@ -382,6 +382,10 @@ def test_matrix_core_tiles_on_any_grid(nu, nv, single, supp):
     both, _ = O.vis2dirty(uvw, freq, cv, rw, single=single, outputs=("dirty", "psf"), **common)
     assert rel_linf(dirty, both["dirty"]) < TOL_ORACLE[single]
     assert rel_linf(psf, both["psf"]) < TOL_ORACLE[single]
+    # degridding from the same tiles (on the matrix cores in double precision)
+    x = np.random.default_rng(nv).standard_normal((nx, ny))
+    got, ref, info, rinfo = d2v(uvw, freq, x, wgt, dx, 1e-3, single, kernel=kernel)
+    assert rel_linf(got, ref) < TOL_ORACLE[single]
 
 
 def test_double_batch_on_the_matrix_cores():
