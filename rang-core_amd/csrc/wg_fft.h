@@ -69,6 +69,39 @@ __host__ __device__ __forceinline__ unsigned udiv(unsigned x, unsigned d, unsign
     return d == 1 ? x : unsigned((unsigned long long)x * m >> 32);
 }
 
+// Host: exp(-2 pi i m / n) for m < n, computed in extended precision on an
+// eighth of the circle (a quarter or half where 4 or 2 are the largest powers
+// of two in n) and mirrored to the rest.
+inline std::vector<double> fft_roots(int n) {
+    std::vector<double> r(std::size_t(2) * n);
+    const long double pi = 3.141592653589793238462643383279502884L;
+    auto set = [&](int m, double c, double s) {
+        r[2 * std::size_t(m)] = c;
+        r[2 * std::size_t(m) + 1] = s;
+    };
+    const int last = n % 8 == 0 ? n / 8 : n % 4 == 0 ? n / 4 : n / 2;
+    for (int m = 0; m <= last && m < n; ++m) {
+        const long double a = 2.0L * pi * (long double)m / (long double)n;
+        set(m, double(cosl(a)), -double(sinl(a)));
+    }
+    // (c, -s) at m: reflected about an eighth, a quarter and a half of the circle
+    if (n % 8 == 0)
+        for (int m = n / 8 + 1; m <= n / 4; ++m) {
+            const std::size_t k = 2 * std::size_t(n / 4 - m);
+            set(m, -r[k + 1], -r[k]);
+        }
+    if (n % 4 == 0)
+        for (int m = n / 4 + 1; m <= n / 2; ++m) {
+            const std::size_t k = 2 * std::size_t(n / 2 - m);
+            set(m, -r[k], r[k + 1]);
+        }
+    for (int m = n / 2 + 1; m < n; ++m) {
+        const std::size_t k = 2 * std::size_t(n - m);
+        set(m, r[k], -r[k + 1]);
+    }
+    return r;
+}
+
 // Host: the passes of length n and its twiddle table (double precision).
 // With fuse21, 3 and 7 together go as one radix-21 pass; such a plan is for
 // the transforms run by fft_lds<..., true> only.
@@ -106,18 +139,17 @@ inline bool fft_describe(int n, FftDesc& d, std::vector<double>& tw_re_im, bool 
         ns *= d.radix[s];
     }
     tw_re_im.assign(std::size_t(2) * (total > 0 ? total : 1), 0.0);
-    const long double pi = 3.141592653589793238462643383279502884L;
+    const std::vector<double> root = fft_roots(n);
     for (int s = 0; s < d.npass; ++s) {
         const int r = d.radix[s];
+        const long long den = (long long)d.ns[s] * r;  // divides n
         for (int k = 0; k < d.ns[s]; ++k)
             for (int t = 1; t < r; ++t) {
                 // reduce k t / (Ns R) to [0, 1) exactly before the angle
-                const long long num = (long long)k * t, den = (long long)d.ns[s] * r;
-                const long double frac = (long double)(num % den) / (long double)den;
-                const long double ang = -2.0L * pi * frac;
+                const std::size_t m = 2 * std::size_t(((long long)k * t) % den * (n / den));
                 const std::size_t at = std::size_t(d.twoff[s] + k * (r - 1) + (t - 1));
-                tw_re_im[2 * at] = double(cosl(ang));
-                tw_re_im[2 * at + 1] = double(sinl(ang));
+                tw_re_im[2 * at] = root[m];
+                tw_re_im[2 * at + 1] = root[m + 1];
             }
     }
     return true;
