@@ -1842,66 +1842,20 @@ __device__ __forceinline__ int table_index(const Geo& g, int i, int j) {
     return min(i, g.nx - i) * g.tny + min(j, g.ny - j);
 }
 
-// The w-screen of plane w at table value s (wgridder.rs:2296-2314).
+// The w-screen exp(+-2 pi i w s) of plane w at table value s
+// (wgridder.rs:2296-2314).
 template <class T>
 __device__ __forceinline__ cx<T> screen_at(double w, double s, bool adjoint) {
     double phs = w * s;
-    if (adjoint) phs = -phs;
-    T ang;
-    if constexpr (sizeof(T) == 4)
-        ang = T(2.0 * M_PI * (phs - floor(phs)));
-    else
-        ang = T(2.0 * M_PI * phs);
     T sn, cs;
-    sincos_t(ang, sn, cs);
-    return {cs, sn};
-}
-
-// Fills LDS from memory with every load of the block in flight before the
-// first LDS write (a transform's loads are otherwise serialised on their
-// latency): element e < count (count <= MT) is src[at(e).first], stored at
-// buf[at(e).second].
-template <class T, int NT, int MT, class At>
-__device__ __forceinline__ void staged_fill(cx<T>* buf, const cx<T>* src, int count, At at) {
-    constexpr int PER = (MT + NT - 1) / NT;
     if constexpr (sizeof(T) == 4) {
-        cx<T> r[PER];
-        int dst[PER];
-#pragma unroll
-        for (int k = 0; k < PER; ++k) {
-            const int e = threadIdx.x + k * NT;
-            if (e < count) {
-                const auto sd = at(e);
-                r[k] = src[sd.first];
-                dst[k] = sd.second;
-            }
-        }
-#pragma unroll
-        for (int k = 0; k < PER; ++k) {
-            const int e = threadIdx.x + k * NT;
-            if (e < count) buf[dst[k]] = r[k];
-        }
+        sincos_turns(phs, sn, cs);
+        if (adjoint) sn = -sn;
     } else {
-        // double: the values staged as two-lane vectors (staging arrays of the
-        // complex struct are placed in scratch memory by the compiler)
-        using V = __attribute__((ext_vector_type(2))) double;
-        V r[PER];
-        int dst[PER];
-#pragma unroll
-        for (int k = 0; k < PER; ++k) {
-            const int e = threadIdx.x + k * NT;
-            if (e < count) {
-                const auto sd = at(e);
-                r[k] = *reinterpret_cast<const V*>(src + sd.first);
-                dst[k] = sd.second;
-            }
-        }
-#pragma unroll
-        for (int k = 0; k < PER; ++k) {
-            const int e = threadIdx.x + k * NT;
-            if (e < count) *reinterpret_cast<V*>(buf + dst[k]) = r[k];
-        }
+        if (adjoint) phs = -phs;
+        sincos_t(T(2.0 * M_PI * phs), sn, cs);
     }
+    return {cs, sn};
 }
 
 // A linear block index remapped so that the workgroups one XCD holds at a time
@@ -1923,6 +1877,90 @@ struct RowOcc {
     const std::uint8_t* occ;  // null: every cell is read
     int G;                    // planes per group
     unsigned mtv;             // udiv multiplier for the tile side Tv
+};
+
+// The ends of a long plane transform (one that fills most of a CU's LDS, so that
+// no second workgroup hides its loads, stores and barriers): the first pass
+// reads memory and the last one writes it, and a value makes two fewer trips
+// through LDS. Lines of 14784 (8192^2 image, 26 planes), columns: inverse
+// 18.3 -> 15.2 ms, forward 18.5 -> 15.7 ms; forward rows 21.2 -> 17.6 ms. Not the inverse
+// rows, which look up each cell's tile first (19.5 -> 22.0 ms), and not where
+// two workgroups or more share a CU (2048^2: the four transforms 1.70 -> 1.73 ms).
+struct None {};
+
+// The image value that lies at u of a grid line of `len` (>= n: none).
+__device__ __forceinline__ int image_of(int u, int len, int n) {
+    const int i = u - (len - n / 2);
+    return i < 0 ? i + len : i;
+}
+
+template <class T>
+struct LineEnd {  // a whole line
+    cx<T>* p;
+    __device__ __forceinline__ None fetch(int, int) const { return {}; }
+    __device__ __forceinline__ cx<T> get(int u0, int du, None) const { return p[u0 + du]; }
+    __device__ __forceinline__ void put(int u0, int du, None, cx<T> v) const { p[u0 + du] = v; }
+};
+
+template <class T>
+struct PaddedIn {  // n values placed on a line of len, zero between
+    const cx<T>* p;
+    int len, n;
+    __device__ __forceinline__ None fetch(int, int) const { return {}; }
+    __device__ __forceinline__ cx<T> get(int u0, int du, None) const {
+        const int j = image_of(u0 + du, len, n);
+        return j < n ? p[j] : cx<T>{T(0), T(0)};
+    }
+};
+
+template <class T>
+struct ProjectOut {  // Re(g screen) of image column j
+    const Geo& g;
+    T* dst;
+    const double* screen;
+    double w0;
+    int j;
+    __device__ __forceinline__ double fetch(int u0, int du) const {
+        const int i = image_of(u0 + du, g.nu, g.nx);
+        return g.wgrid && i < g.nx ? screen[table_index(g, i, j)] : 0.0;
+    }
+    __device__ __forceinline__ void put(int u0, int du, double s, cx<T> v) const {
+        const int i = image_of(u0 + du, g.nu, g.nx);
+        if (i >= g.nx) return;
+        T term = v.re;
+        if (g.wgrid) {
+            const cx<T> ph = screen_at<T>(w0, s, true);
+            term = v.re * ph.re - v.im * ph.im;
+        }
+        dst[g.cm ? (long long)j * g.nx + i : (long long)i * g.ny + j] = term;
+    }
+};
+
+template <class T>
+struct ImageIn {  // image column j times the screen, zero beyond the image
+    struct P {
+        T v;
+        double s;
+    };
+    const Geo& g;
+    const T* img;
+    const double* screen;
+    double w0;
+    int j;
+    __device__ __forceinline__ P fetch(int u0, int du) const {
+        const int i = image_of(u0 + du, g.nu, g.nx);
+        P p{T(0), 0.0};
+        if (i < g.nx) {
+            p.v = img[g.cm ? (long long)j * g.nx + i : (long long)i * g.ny + j];
+            if (g.wgrid) p.s = screen[table_index(g, i, j)];
+        }
+        return p;
+    }
+    __device__ __forceinline__ cx<T> get(int u0, int du, P p) const {
+        if (!g.wgrid || image_of(u0 + du, g.nu, g.nx) >= g.nx) return {p.v, T(0)};
+        const cx<T> ph = screen_at<T>(w0, p.s, false);
+        return {p.v * ph.re, p.v * ph.im};
+    }
 };
 
 // v2d: inverse transform along v of one grid row, keeping the image columns
@@ -1995,7 +2033,7 @@ __global__ __launch_bounds__(NT) void k_rows_inv(const cx<T>* __restrict__ grid,
         for (int j = threadIdx.x; j < ny; j += NT) tmp[row * ny + j] = cx<T>{T(0), T(0)};
         return;
     }
-    fft_lds<T, NT, MAXTOT, sizeof(T) == 4>(buf, d, 1, tw, +1);
+    fft_lds<T, NT, MAXTOT, +1, sizeof(T) == 4>(buf, d, 1, tw);
     const int sh = nv - ny / 2;
     for (int j = threadIdx.x; j < ny; j += NT) {
         const int e = sh + j;
@@ -2020,6 +2058,14 @@ __global__ __launch_bounds__(NT) void k_cols_inv(const cx<T>* __restrict__ tmp,
     const int p = lin / ncb;
     const int j0 = (lin - p * ncb) * C, nc = min(C, ny - j0);
     const cx<T>* src = tmp + (long long)p * nu * ny;
+    if constexpr (SCM && NT == 1024) {
+        if (nc == 1 && d.npass > 1) {
+            fft_ends<T, NT, MAXTOT, +1>(
+                buf, d, tw, LineEnd<T>{const_cast<cx<T>*>(src) + (long long)j0 * nu},
+                ProjectOut<T>{g, proj + (long long)p * nx * ny, screen, g.wmin + double(p) * g.dw, j0});
+            return;
+        }
+    }
     const unsigned mnc = nc > 1 ? unsigned(((1ull << 32) + nc - 1) / nc) : 0u;
     // nu * nc <= MAXTOT
     if constexpr (SCM) {
@@ -2033,7 +2079,7 @@ __global__ __launch_bounds__(NT) void k_cols_inv(const cx<T>* __restrict__ tmp,
         });
     }
     __syncthreads();
-    fft_lds<T, NT, MAXTOT, sizeof(T) == 4>(buf, d, nc, tw, +1);
+    fft_lds<T, NT, MAXTOT, +1, sizeof(T) == 4>(buf, d, nc, tw);
     const double w0 = g.wmin + double(p) * g.dw;
     T* dst = proj + (long long)p * nx * ny;
     const int sh = nu - nx / 2;
@@ -2199,6 +2245,13 @@ __global__ __launch_bounds__(NT) void k_cols_fwd(const T* __restrict__ img,
     const int lin = xcd_remap(blockIdx.x, gridDim.x);
     const int p = lin / ncb;
     const int j0 = (lin - p * ncb) * C, nc = min(C, ny - j0);
+    if constexpr (TCM && NT == 1024) {
+        if (nc == 1 && d.npass > 1) {
+            fft_ends<T, NT, MAXTOT, -1>(buf, d, tw, ImageIn<T>{g, img, screen, g.wmin + double(p) * g.dw, j0},
+                                        LineEnd<T>{tmp + ((long long)p * ny + j0) * nu});
+            return;
+        }
+    }
     const unsigned mnc = nc > 1 ? unsigned(((1ull << 32) + nc - 1) / nc) : 0u;
     // the image values of the block in flight while the buffer is cleared
     constexpr int PER = (MAXTOT + NT - 1) / NT;
@@ -2248,7 +2301,7 @@ __global__ __launch_bounds__(NT) void k_cols_fwd(const T* __restrict__ img,
         }
     }
     __syncthreads();
-    fft_lds<T, NT, MAXTOT, sizeof(T) == 4>(buf, d, nc, tw, -1);
+    fft_lds<T, NT, MAXTOT, -1, sizeof(T) == 4>(buf, d, nc, tw);
     cx<T>* dst = tmp + (long long)p * nu * ny;
     if constexpr (TCM) {
         for (int e = threadIdx.x; e < nu * nc; e += NT) dst[(long long)j0 * nu + e] = buf[e];
@@ -2275,13 +2328,21 @@ __global__ __launch_bounds__(NT) void k_rows_fwd(const cx<T>* __restrict__ tmp,
     // a row no degridding item reads is neither transformed nor written
     if (need && !need[row - p * g.nu]) return;
     const long long src = p * g.nu + upos(g, int(row - p * g.nu));
+    if constexpr (NT == 1024) {
+        if (d.npass > 1) {
+            fft_ends<T, NT, MAXTOT, -1>(buf, d, tw, PaddedIn<T>{tmp + src * ny, nv, ny}, LineEnd<T>{grid + row * nv});
+            return;
+        }
+    }
     // the image row in flight while the buffer is cleared
     constexpr int PER = (MAXTOT + NT - 1) / NT;
-    cx<T> r[PER];
+    // double: a staging array of the complex struct goes to scratch memory
+    using V = std::conditional_t<sizeof(T) == 4, cx<T>, typename Lds<T>::pair>;
+    V r[PER];
 #pragma unroll
     for (int k = 0; k < PER; ++k) {
         const int j = threadIdx.x + k * NT;
-        if (j < ny) r[k] = tmp[src * ny + j];
+        if (j < ny) r[k] = *reinterpret_cast<const V*>(tmp + src * ny + j);
     }
     for (int e = threadIdx.x; e < nv; e += NT) buf[e] = cx<T>{T(0), T(0)};
     __syncthreads();
@@ -2291,11 +2352,11 @@ __global__ __launch_bounds__(NT) void k_rows_fwd(const cx<T>* __restrict__ tmp,
         const int j = threadIdx.x + k * NT;
         if (j < ny) {
             const int e = sh + j;
-            buf[e >= nv ? e - nv : e] = r[k];
+            *reinterpret_cast<V*>(buf + (e >= nv ? e - nv : e)) = r[k];
         }
     }
     __syncthreads();
-    fft_lds<T, NT, MAXTOT, sizeof(T) == 4>(buf, d, 1, tw, -1);
+    fft_lds<T, NT, MAXTOT, -1, sizeof(T) == 4>(buf, d, 1, tw);
     cx<T>* dst = grid + row * nv;
     for (int e = threadIdx.x; e < nv; e += NT) dst[e] = buf[e];
 }
@@ -2331,7 +2392,7 @@ __global__ __launch_bounds__(NT) void k_lrow_p1(cx<T>* data, int n1, int n2, int
         return std::pair<long long, int>((long long)j1 * n2 + j20 + c, c * n1 + j1);
     });
     __syncthreads();
-    fft_lds<T, NT, MT>(buf, d1, nc, tw1, sgn);
+    fft_lds_either<T, NT, MT>(buf, d1, nc, tw1, sgn);
     for (int e = threadIdx.x; e < n1 * nc; e += NT) {
         const int k1 = e / nc, c = e - k1 * nc;
         x[(long long)k1 * n2 + j20 + c] = cmul(buf[c * n1 + k1], twn_at(twn, (j20 + c) * k1, sgn));
@@ -2353,7 +2414,7 @@ __global__ __launch_bounds__(NT) void k_lrow_p2(cx<T>* data, int n1, int n2, int
     staged_fill<T, NT, MT>(buf, x, n2 * nc,
                            [&](int e) { return std::pair<long long, int>((long long)k10 * n2 + e, e); });
     __syncthreads();
-    fft_lds<T, NT, MT>(buf, d2, nc, tw2, sgn);
+    fft_lds_either<T, NT, MT>(buf, d2, nc, tw2, sgn);
     for (int e = threadIdx.x; e < n2 * nc; e += NT) {
         const int c = e / n2, k2 = e - c * n2;
         if constexpr (MODE == 0) {
@@ -2385,7 +2446,7 @@ __global__ __launch_bounds__(NT) void k_lcol_p1(cx<T>* data, int n1, int n2, int
         return std::pair<long long, int>(((long long)j1 * n2 + j20 + c2) * M + m0 + cm, r * n1 + j1);
     });
     __syncthreads();
-    fft_lds<T, NT, MT>(buf, d1, lines, tw1, sgn);
+    fft_lds_either<T, NT, MT>(buf, d1, lines, tw1, sgn);
     for (int e = threadIdx.x; e < n1 * lines; e += NT) {
         const int k1 = e / lines, r = e - k1 * lines, c2 = r / ncm, cm = r - c2 * ncm;
         x[((long long)k1 * n2 + j20 + c2) * M + m0 + cm] = cmul(buf[r * n1 + k1], twn_at(twn, (j20 + c2) * k1, sgn));
@@ -2413,7 +2474,7 @@ __global__ __launch_bounds__(NT) void k_lcol_p2(cx<T>* data, int n1, int n2, int
         return std::pair<long long, int>(((long long)(k10 + c1) * n2 + j2) * M + m0 + cm, r * n2 + j2);
     });
     __syncthreads();
-    fft_lds<T, NT, MT>(buf, d2, lines, tw2, sgn);
+    fft_lds_either<T, NT, MT>(buf, d2, lines, tw2, sgn);
     const double w0 = g.wmin + double(p) * g.dw;
     for (int e = threadIdx.x; e < n2 * lines; e += NT) {
         const int k2 = e / lines, r = e - k2 * lines, c1 = r / ncm, cm = r - c1 * ncm;

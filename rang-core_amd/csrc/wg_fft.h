@@ -11,6 +11,7 @@
 // table in global memory computed on the host in double precision.
 #pragma once
 
+#include <type_traits>
 #include <hip/hip_runtime.h>
 
 #include <vector>
@@ -21,8 +22,10 @@ namespace rang {
 
 constexpr int kFftMaxPass = 24;
 
+// Aligned as a pair, so that a value moves through LDS in one 8- or 16-byte
+// access (two 4-byte ones at a stride of 8 bytes use every other bank).
 template <class T>
-struct cx {
+struct alignas(2 * sizeof(T)) cx {
     T re, im;
 };
 
@@ -38,10 +41,10 @@ template <class T>
 __device__ __forceinline__ cx<T> csub(cx<T> a, cx<T> b) {
     return {a.re - b.re, a.im - b.im};
 }
-// (sgn i) * a
-template <class T>
-__device__ __forceinline__ cx<T> cmul_si(cx<T> a, int sgn) {
-    return sgn > 0 ? cx<T>{-a.im, a.re} : cx<T>{a.im, -a.re};
+// (SGN i) * a
+template <int SGN, class T>
+__device__ __forceinline__ cx<T> cmul_si(cx<T> a) {
+    return SGN > 0 ? cx<T>{-a.im, a.re} : cx<T>{a.im, -a.re};
 }
 
 // Passes of one length: radix, stride Ns before the pass and offset of the
@@ -61,7 +64,7 @@ struct FftDesc {
 // x / d as the high half of x * ceil(2^32 / d), exact for x, d < 2^16 (every
 // index here is below the transform length). d = 1 has no 32-bit multiplier
 // (it would be 2^32) and is taken apart.
-inline unsigned fft_magic(unsigned d) {
+__host__ __device__ inline unsigned fft_magic(unsigned d) {
     return d <= 1 ? 0u : unsigned(((1ull << 32) + d - 1) / d);
 }
 
@@ -155,7 +158,8 @@ inline bool fft_describe(int n, FftDesc& d, std::vector<double>& tw_re_im, bool 
     return true;
 }
 
-// Small DFTs, out[q] = sum_t v[t] exp(sgn 2 pi i t q / R), in place.
+// Small DFTs, out[q] = sum_t v[t] exp(SGN 2 pi i t q / R), in place; SGN (+1 or
+// -1) is a template argument, so signs fold into the instructions.
 template <class T>
 __device__ __forceinline__ void dft2(cx<T>* v) {
     cx<T> a = v[0], b = v[1];
@@ -163,10 +167,10 @@ __device__ __forceinline__ void dft2(cx<T>* v) {
     v[1] = csub(a, b);
 }
 
-template <class T>
-__device__ __forceinline__ void dft4(cx<T>* v, int sgn) {
+template <int SGN, class T>
+__device__ __forceinline__ void dft4(cx<T>* v) {
     cx<T> t0 = cadd(v[0], v[2]), t1 = csub(v[0], v[2]);
-    cx<T> t2 = cadd(v[1], v[3]), t3 = cmul_si(csub(v[1], v[3]), sgn);
+    cx<T> t2 = cadd(v[1], v[3]), t3 = cmul_si<SGN>(csub(v[1], v[3]));
     v[0] = cadd(t0, t2);
     v[2] = csub(t0, t2);
     v[1] = cadd(t1, t3);
@@ -174,29 +178,29 @@ __device__ __forceinline__ void dft4(cx<T>* v, int sgn) {
 }
 
 // out[2q] = DFT4(x_t + x_{t+4}), out[2q+1] = DFT4((x_t - x_{t+4}) W8^t).
-template <class T>
-__device__ __forceinline__ void dft8(cx<T>* v, int sgn) {
+template <int SGN, class T>
+__device__ __forceinline__ void dft8(cx<T>* v) {
     const T h = T(0.70710678118654752440084436210484903928);
     cx<T> a[4], b[4];
     for (int t = 0; t < 4; ++t) {
         a[t] = cadd(v[t], v[t + 4]);
         b[t] = csub(v[t], v[t + 4]);
     }
-    // W8^1 = h (1 + sgn i), W8^2 = sgn i, W8^3 = h (-1 + sgn i)
-    b[1] = cmul(b[1], cx<T>{h, T(sgn) * h});
-    b[2] = cmul_si(b[2], sgn);
-    b[3] = cmul(b[3], cx<T>{-h, T(sgn) * h});
-    dft4(a, sgn);
-    dft4(b, sgn);
+    // W8^1 = h (1 + SGN i), W8^2 = SGN i, W8^3 = h (-1 + SGN i)
+    b[1] = cmul(b[1], cx<T>{h, T(SGN) * h});
+    b[2] = cmul_si<SGN>(b[2]);
+    b[3] = cmul(b[3], cx<T>{-h, T(SGN) * h});
+    dft4<SGN>(a);
+    dft4<SGN>(b);
     for (int q = 0; q < 4; ++q) {
         v[2 * q] = a[q];
         v[2 * q + 1] = b[q];
     }
 }
 
-// Odd R: pairs (t, R - t) give out[q] = v0 + sum a_t cos + sgn i sum b_t sin.
-template <class T, int R>
-__device__ __forceinline__ void dft_odd(cx<T>* v, int sgn) {
+// Odd R: pairs (t, R - t) give out[q] = v0 + sum a_t cos + SGN i sum b_t sin.
+template <class T, int R, int SGN>
+__device__ __forceinline__ void dft_odd(cx<T>* v) {
     constexpr int m = (R - 1) / 2;
     const double* cs = R == 3 ? kCos3 : R == 5 ? kCos5 : R == 7 ? kCos7 : kCos11;
     const double* sn = R == 3 ? kSin3 : R == 5 ? kSin5 : R == 7 ? kSin7 : kSin11;
@@ -219,7 +223,7 @@ __device__ __forceinline__ void dft_odd(cx<T>* v, int sgn) {
             A = {A.re + a[t].re * c, A.im + a[t].im * c};
             B = {B.re + b[t].re * s, B.im + b[t].im * s};
         }
-        const cx<T> iB = cmul_si(B, sgn);
+        const cx<T> iB = cmul_si<SGN>(B);
         out[q] = cadd(A, iB);
         out[R - q] = csub(A, iB);
     }
@@ -231,8 +235,8 @@ __device__ __forceinline__ void dft_odd(cx<T>* v, int sgn) {
 // so no twiddles between its two stages: a[n1][n2] = v[(7 n1 + 3 n2) mod 21],
 // DFT3 along n1, DFT7 along n2, out[(7 k1 + 15 k2) mod 21] = a[k1][k2]. One
 // pass (and its two barriers) fewer wherever 3 and 7 both divide a length.
-template <class T>
-__device__ __forceinline__ void dft21(cx<T>* v, int sgn) {
+template <int SGN, class T>
+__device__ __forceinline__ void dft21(cx<T>* v) {
     cx<T> a[3][7];
 #pragma unroll
     for (int n1 = 0; n1 < 3; ++n1)
@@ -241,31 +245,54 @@ __device__ __forceinline__ void dft21(cx<T>* v, int sgn) {
 #pragma unroll
     for (int n2 = 0; n2 < 7; ++n2) {
         cx<T> c[3] = {a[0][n2], a[1][n2], a[2][n2]};
-        dft_odd<T, 3>(c, sgn);
+        dft_odd<T, 3, SGN>(c);
 #pragma unroll
         for (int k1 = 0; k1 < 3; ++k1) a[k1][n2] = c[k1];
     }
 #pragma unroll
     for (int k1 = 0; k1 < 3; ++k1) {
-        dft_odd<T, 7>(a[k1], sgn);
+        dft_odd<T, 7, SGN>(a[k1]);
 #pragma unroll
         for (int k2 = 0; k2 < 7; ++k2) v[(7 * k1 + 15 * k2) % 21] = a[k1][k2];
     }
 }
 
-template <class T, int R>
-__device__ __forceinline__ void dft_small(cx<T>* v, int sgn) {
+template <class T, int R, int SGN>
+__device__ __forceinline__ void dft_small(cx<T>* v) {
     if constexpr (R == 2)
         dft2(v);
     else if constexpr (R == 4)
-        dft4(v, sgn);
+        dft4<SGN>(v);
     else if constexpr (R == 8)
-        dft8(v, sgn);
+        dft8<SGN>(v);
     else if constexpr (R == 21)
-        dft21(v, sgn);
+        dft21<SGN>(v);
     else
-        dft_odd<T, R>(v, sgn);
+        dft_odd<T, R, SGN>(v);
 }
+
+// A value's place in LDS as a 32-bit address, and the place `step` values further
+// on by one addition (opaque to the optimiser, which would otherwise form each
+// position anew from the first).
+template <class T>
+struct Lds {
+    typedef T pair __attribute__((ext_vector_type(2)));
+    typedef __attribute__((address_space(3))) pair* ptr;
+};
+template <class P>
+__device__ __forceinline__ P lds_step(P p, int step) {
+    p += step;
+    asm("" : "+v"(p));
+    return p;
+}
+
+// Where a pass takes its values from and leaves them. Plain LDS is LdsEnd; any
+// other end (of a single transform) is a pair of calls per value, `fetch` (every
+// load of the pass, all in flight before the first use) and then `get` or `put`:
+//   P fetch(u0, du)         for value u0 + du of the transform; du is uniform
+//   cx get(u0, du, P)       the value to transform
+//   void put(u0, du, P, v)  the value transformed
+struct LdsEnd {};
 
 // One Stockham pass of radix R over `ncol` transforms of length n in LDS.
 // BMAX bounds the butterflies per thread (ceil(ncol n / (R NT))). With ONE
@@ -276,87 +303,177 @@ __device__ __forceinline__ void dft_small(cx<T>* v, int sgn) {
 // multiply-high, quarter-rate on the VALU. Several transforms recompute their
 // indices in the store phase instead, which keeps no index registers live
 // across the barrier (their kernels hold two transforms' registers).
-template <class T, int NT, int R, int BMAX, bool ONE>
-__device__ __forceinline__ void fft_pass(cx<T>* buf, int n, int ncol, int ns, unsigned mnb,
-                                         unsigned mns, const cx<T>* tw, int sgn) {
+// The passes are bound by the VALU (97 % busy in 2048^2 column transforms), so
+// the direction is a template argument (no sign selects) and LDS addresses step
+// by nb and ns in 32-bit additions: 16.4 -> 14.2 VALU instructions a value and
+// pass at radix 8, 24.5 -> 21.3 at radix 21.
+template <class T, int NT, int R, int BMAX, bool ONE, int SGN, class In, class Out>
+__device__ __forceinline__ void fft_pass(cx<T>* buf, int n, int ncol, int ns, unsigned mnb, unsigned mns,
+                                         const cx<T>* tw, In& in, Out& out) {
+    constexpr bool SRC = !std::is_same_v<In, LdsEnd>, DST = !std::is_same_v<Out, LdsEnd>;
     const int nb = n / R;
     const int total = ONE ? nb : nb * ncol;
+    static_assert(ONE || !(SRC || DST));
+    // butterfly j: its transform and its number within it
+    auto place = [&](int j, int& c, int& jj) {
+        c = 0;
+        jj = j;
+        if constexpr (!ONE) {
+            c = int(udiv(unsigned(j), unsigned(nb), mnb));
+            jj = j - c * nb;
+        }
+    };
+    // its first output value within the transform, and its twiddle
+    auto first_of = [&](int jj, int& k) {
+        const int q = int(udiv(unsigned(jj), unsigned(ns), mns));
+        k = jj - q * ns;
+        return q * ns * R + k;
+    };
     cx<T> v[BMAX][R];
     int cb[ONE ? BMAX : 1];
+    if constexpr (SRC) {
+        using P = decltype(in.fetch(0, 0));
+        P pre[BMAX][R];
+#pragma unroll
+        for (int b = 0; b < BMAX; ++b) {
+            const int j = int(threadIdx.x) + b * NT;
+            if (j < total) {
+                int c, jj;
+                place(j, c, jj);
+#pragma unroll
+                for (int t = 0; t < R; ++t) pre[b][t] = in.fetch(jj, t * nb);
+            }
+        }
+#pragma unroll
+        for (int b = 0; b < BMAX; ++b) {
+            const int j = int(threadIdx.x) + b * NT;
+            if (j < total) {
+                int c, jj;
+                place(j, c, jj);
+#pragma unroll
+                for (int t = 0; t < R; ++t) v[b][t] = in.get(jj, t * nb, pre[b][t]);
+            }
+        }
+    }
 #pragma unroll
     for (int b = 0; b < BMAX; ++b) {
         const int j = int(threadIdx.x) + b * NT;
         if (j < total) {
-            int c = 0, jj = j;
-            if constexpr (!ONE) {
-                c = int(udiv(unsigned(j), unsigned(nb), mnb));
-                jj = j - c * nb;
-            }
-            const cx<T>* col = buf + c * n;
+            int c, jj, k = 0;
+            place(j, c, jj);
+            if constexpr (!SRC) {
+                typename Lds<T>::ptr from = (typename Lds<T>::ptr)buf + (c * n + jj);
 #pragma unroll
-            for (int t = 0; t < R; ++t) v[b][t] = col[jj + t * nb];
-            int k = 0;
-            if constexpr (ONE) {
-                const int q = int(udiv(unsigned(jj), unsigned(ns), mns));
-                k = jj - q * ns;
-                cb[b] = q * ns * R + k;
-            } else if (ns > 1) {
-                k = jj - int(udiv(unsigned(jj), unsigned(ns), mns)) * ns;
+                for (int t = 0; t < R; ++t) {
+                    v[b][t] = {from->x, from->y};
+                    from = lds_step(from, nb);
+                }
             }
-            if (ns > 1) {
+            if constexpr (ONE)
+                cb[b] = first_of(jj, k);
+            else if (!SRC && ns > 1)
+                first_of(jj, k);
+            if (!SRC && ns > 1) {  // the first pass has no twiddles
                 const cx<T>* w = tw + k * (R - 1);
 #pragma unroll
                 for (int t = 1; t < R; ++t) {
                     cx<T> f = w[t - 1];
-                    if (sgn > 0) f.im = -f.im;
+                    if (SGN > 0) f.im = -f.im;
                     v[b][t] = cmul(v[b][t], f);
                 }
             }
-            dft_small<T, R>(v[b], sgn);
+            dft_small<T, R, SGN>(v[b]);
         }
     }
-    __syncthreads();
+    if constexpr (DST) {
+        using P = decltype(out.fetch(0, 0));
+        P pre[BMAX][R];
 #pragma unroll
-    for (int b = 0; b < BMAX; ++b) {
-        const int j = int(threadIdx.x) + b * NT;
-        if (j < total) {
-            int base;
-            cx<T>* col = buf;
-            if constexpr (ONE) {
-                base = cb[b];
-            } else {
-                const int c = int(udiv(unsigned(j), unsigned(nb), mnb)), jj = j - c * nb;
-                const int q = int(udiv(unsigned(jj), unsigned(ns), mns)), k = jj - q * ns;
-                col = buf + c * n;
-                base = q * ns * R + k;
+        for (int b = 0; b < BMAX; ++b) {
+            const int j = int(threadIdx.x) + b * NT;
+            if (j < total) {
+                int c, jj, k;
+                place(j, c, jj);
+                const int base = ONE ? cb[ONE ? b : 0] : first_of(jj, k);
+#pragma unroll
+                for (int t = 0; t < R; ++t) pre[b][t] = out.fetch(base, t * ns);
             }
-#pragma unroll
-            for (int t = 0; t < R; ++t) col[base + t * ns] = v[b][t];
         }
+#pragma unroll
+        for (int b = 0; b < BMAX; ++b) {
+            const int j = int(threadIdx.x) + b * NT;
+            if (j < total) {
+                int c, jj, k;
+                place(j, c, jj);
+                const int base = ONE ? cb[ONE ? b : 0] : first_of(jj, k);
+#pragma unroll
+                for (int t = 0; t < R; ++t) out.put(base, t * ns, pre[b][t], v[b][t]);
+            }
+        }
+    } else {
+        if constexpr (!SRC) __syncthreads();  // every value read
+#pragma unroll
+        for (int b = 0; b < BMAX; ++b) {
+            const int j = int(threadIdx.x) + b * NT;
+            if (j < total) {
+                int c, jj, k;
+                place(j, c, jj);
+                const int base = ONE ? cb[ONE ? b : 0] : first_of(jj, k);
+                typename Lds<T>::ptr to = (typename Lds<T>::ptr)buf + (c * n + base);
+#pragma unroll
+                for (int t = 0; t < R; ++t) {
+                    to->x = v[b][t].re;
+                    to->y = v[b][t].im;
+                    to = lds_step(to, ns);
+                }
+            }
+        }
+        __syncthreads();
     }
-    __syncthreads();
 }
 
 constexpr int cdiv(int a, int b) { return (a + b - 1) / b; }
 
-template <class T, int NT, int MAXTOT, bool ONE, bool R21>
-__device__ void fft_passes(cx<T>* buf, const FftDesc& d, int ncol, const cx<T>* tw, int sgn) {
-    for (int s = 0; s < d.npass; ++s) {
-        const cx<T>* tws = tw + d.twoff[s];
-        const unsigned a = d.mnb[s], b = d.mns[s];
-        switch (d.radix[s]) {
-        case 2: fft_pass<T, NT, 2, cdiv(MAXTOT, 2 * NT), ONE>(buf, d.n, ncol, d.ns[s], a, b, tws, sgn); break;
-        case 3: fft_pass<T, NT, 3, cdiv(MAXTOT, 3 * NT), ONE>(buf, d.n, ncol, d.ns[s], a, b, tws, sgn); break;
-        case 4: fft_pass<T, NT, 4, cdiv(MAXTOT, 4 * NT), ONE>(buf, d.n, ncol, d.ns[s], a, b, tws, sgn); break;
-        case 5: fft_pass<T, NT, 5, cdiv(MAXTOT, 5 * NT), ONE>(buf, d.n, ncol, d.ns[s], a, b, tws, sgn); break;
-        case 7: fft_pass<T, NT, 7, cdiv(MAXTOT, 7 * NT), ONE>(buf, d.n, ncol, d.ns[s], a, b, tws, sgn); break;
-        case 8: fft_pass<T, NT, 8, cdiv(MAXTOT, 8 * NT), ONE>(buf, d.n, ncol, d.ns[s], a, b, tws, sgn); break;
-        case 21:
-            if constexpr (R21) fft_pass<T, NT, 21, cdiv(MAXTOT, 21 * NT), ONE>(buf, d.n, ncol, d.ns[s], a, b, tws, sgn);
-            break;
-        default: fft_pass<T, NT, 11, cdiv(MAXTOT, 11 * NT), ONE>(buf, d.n, ncol, d.ns[s], a, b, tws, sgn); break;
-        }
+// Pass s of `d`.
+template <class T, int NT, int MAXTOT, bool ONE, bool R21, int SGN, class In, class Out>
+__device__ __forceinline__ void fft_pass_of(cx<T>* buf, const FftDesc& d, int s, int ncol, const cx<T>* tw, In& in,
+                                            Out& out) {
+    const cx<T>* tws = tw + d.twoff[s];
+    const unsigned a = d.mnb[s], b = d.mns[s];
+    const int ns = d.ns[s];
+#define FFT_PASS(R) \
+    fft_pass<T, NT, R, cdiv(MAXTOT, R * NT), ONE, SGN>(buf, d.n, ncol, ns, a, b, tws, in, out)
+    switch (d.radix[s]) {
+    case 2: FFT_PASS(2); break;
+    case 3: FFT_PASS(3); break;
+    case 4: FFT_PASS(4); break;
+    case 5: FFT_PASS(5); break;
+    case 7: FFT_PASS(7); break;
+    case 8: FFT_PASS(8); break;
+    case 21:
+        if constexpr (R21) FFT_PASS(21);
+        break;
+    default: FFT_PASS(11); break;
     }
+#undef FFT_PASS
+}
+
+template <class T, int NT, int MAXTOT, bool ONE, bool R21, int SGN>
+__device__ __forceinline__ void fft_passes(cx<T>* buf, const FftDesc& d, int ncol, const cx<T>* tw) {
+    LdsEnd lds;
+    for (int s = 0; s < d.npass; ++s)
+        fft_pass_of<T, NT, MAXTOT, ONE, R21, SGN>(buf, d, s, ncol, tw, lds, lds);
+}
+
+// One single-precision plane transform of two passes or more, the first from
+// `in` and the last to `out`; the buffer holds nothing on entry.
+template <class T, int NT, int MAXTOT, int SGN, class In, class Out>
+__device__ __forceinline__ void fft_ends(cx<T>* buf, const FftDesc& d, const cx<T>* tw, In in, Out out) {
+    LdsEnd lds;
+    fft_pass_of<T, NT, MAXTOT, true, true, SGN>(buf, d, 0, 1, tw, in, lds);
+    for (int s = 1; s < d.npass - 1; ++s)
+        fft_pass_of<T, NT, MAXTOT, true, true, SGN>(buf, d, s, 1, tw, lds, lds);
+    fft_pass_of<T, NT, MAXTOT, true, true, SGN>(buf, d, d.npass - 1, 1, tw, lds, out);
 }
 
 // All passes of `d` over ncol * d.n <= MAXTOT values in LDS (synchronised
@@ -366,16 +483,97 @@ __device__ void fft_passes(cx<T>* buf, const FftDesc& d, int ncol, const cx<T>* 
 // Other kernels keep one pass form: the extra code would take registers they
 // do not have to spare (the surrogate's column kernels, two transforms each,
 // spilled with it).
-template <class T, int NT, int MAXTOT, bool PLANE = false>
-__device__ void fft_lds(cx<T>* buf, const FftDesc& d, int ncol, const cx<T>* tw, int sgn) {
+template <class T, int NT, int MAXTOT, int SGN, bool PLANE = false>
+__device__ __forceinline__ void fft_lds(cx<T>* buf, const FftDesc& d, int ncol, const cx<T>* tw) {
     if constexpr (PLANE) {
         if (ncol == 1)
-            fft_passes<T, NT, MAXTOT, true, true>(buf, d, 1, tw, sgn);
+            fft_passes<T, NT, MAXTOT, true, true, SGN>(buf, d, 1, tw);
         else
-            fft_passes<T, NT, MAXTOT, false, true>(buf, d, ncol, tw, sgn);
+            fft_passes<T, NT, MAXTOT, false, true, SGN>(buf, d, ncol, tw);
     } else {
-        fft_passes<T, NT, MAXTOT, false, false>(buf, d, ncol, tw, sgn);
+        fft_passes<T, NT, MAXTOT, false, false, SGN>(buf, d, ncol, tw);
     }
+}
+
+// The same with the direction a launch argument.
+template <class T, int NT, int MAXTOT>
+__device__ __forceinline__ void fft_lds_either(cx<T>* buf, const FftDesc& d, int ncol, const cx<T>* tw, int sgn) {
+    if (sgn > 0)
+        fft_lds<T, NT, MAXTOT, +1>(buf, d, ncol, tw);
+    else
+        fft_lds<T, NT, MAXTOT, -1>(buf, d, ncol, tw);
+}
+
+// Fills LDS from memory with every load of the block in flight before the
+// first LDS write (a transform's loads are otherwise serialised on their
+// latency): element e < count (count <= MT) is src[at(e).first], stored at
+// buf[at(e).second].
+template <class T, int NT, int MT, class At>
+__device__ __forceinline__ void staged_fill(cx<T>* buf, const cx<T>* src, int count, At at) {
+    constexpr int PER = (MT + NT - 1) / NT;
+    if constexpr (sizeof(T) == 4) {
+        cx<T> r[PER];
+        int dst[PER];
+#pragma unroll
+        for (int k = 0; k < PER; ++k) {
+            const int e = threadIdx.x + k * NT;
+            if (e < count) {
+                const auto sd = at(e);
+                r[k] = src[sd.first];
+                dst[k] = sd.second;
+            }
+        }
+#pragma unroll
+        for (int k = 0; k < PER; ++k) {
+            const int e = threadIdx.x + k * NT;
+            if (e < count) buf[dst[k]] = r[k];
+        }
+    } else {
+        // double: the values staged as two-lane vectors (staging arrays of the
+        // complex struct are placed in scratch memory by the compiler)
+        using V = __attribute__((ext_vector_type(2))) double;
+        V r[PER];
+        int dst[PER];
+#pragma unroll
+        for (int k = 0; k < PER; ++k) {
+            const int e = threadIdx.x + k * NT;
+            if (e < count) {
+                const auto sd = at(e);
+                r[k] = *reinterpret_cast<const V*>(src + sd.first);
+                dst[k] = sd.second;
+            }
+        }
+#pragma unroll
+        for (int k = 0; k < PER; ++k) {
+            const int e = threadIdx.x + k * NT;
+            if (e < count) *reinterpret_cast<V*>(buf + dst[k]) = r[k];
+        }
+    }
+}
+
+// Single-precision sine and cosine of `turns` whole turns: the whole turns and
+// the nearest quarter turn are taken off in double precision; what is left, at
+// most an eighth of a turn, goes through the Taylor series (first terms left
+// out: x^11 / 11! < 2e-9, x^12 / 12! < 2e-10 at pi / 4). Largest error 8.5e-8;
+// the angle rounded to single precision on up to 2 pi and sincosf: 2.8e-7.
+__device__ __forceinline__ void sincos_turns(double turns, float& sn, float& cs) {
+    const double t = 4.0 * (turns - floor(turns)), qd = rint(t);
+    const int q = int(qd);
+    const float x = float((t - qd) * 1.5707963267948966), z = x * x;
+    float a = fmaf(z, 1.0f / 362880, -1.0f / 5040);
+    a = fmaf(z, a, 1.0f / 120);
+    a = fmaf(z, a, -1.0f / 6);
+    a = fmaf(z * x, a, x);
+    float b = fmaf(z, -1.0f / 3628800, 1.0f / 40320);
+    b = fmaf(z, b, -1.0f / 720);
+    b = fmaf(z, b, 1.0f / 24);
+    b = fmaf(z, b, -0.5f);
+    b = fmaf(z, b, 1.0f);
+    // quarter turns: (c, s), (-s, c), (-c, -s), (s, -c)
+    cs = (q & 1) ? a : b;
+    sn = (q & 1) ? b : a;
+    if ((q + 1) & 2) cs = -cs;
+    if (q & 2) sn = -sn;
 }
 
 // Plane-wise transpose of complex values, [P][R][C] -> [P][C][R], through

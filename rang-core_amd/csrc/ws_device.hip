@@ -562,7 +562,7 @@ __global__ __launch_bounds__(NT) void k_rows(cx<T>* data, FftDesc d, const cx<T>
     cx<T>* row = data + (long long)blockIdx.x * d.n;
     for (int e = threadIdx.x; e < d.n; e += NT) buf[e] = row[e];
     __syncthreads();
-    fft_lds<T, NT, MT>(buf, d, 1, tw, +1);
+    fft_lds<T, NT, MT, +1>(buf, d, 1, tw);
     for (int e = threadIdx.x; e < d.n; e += NT) row[e] = buf[e];
 }
 
@@ -591,7 +591,7 @@ __global__ __launch_bounds__(NT) void k_cols(cx<T>* data, FftDesc d, const cx<T>
         buf[c * H + y] = base[(long long)y * W + x0 + c];
     }
     __syncthreads();
-    fft_lds<T, NT, MT>(buf, d, nc, tw, +1);
+    fft_lds<T, NT, MT, +1>(buf, d, nc, tw);
     for (int e = threadIdx.x; e < H * nc; e += NT) {
         const int y = e / nc, c = e - y * nc;
         base[(long long)y * W + x0 + c] = buf[c * H + y];

@@ -50,7 +50,7 @@ __global__ __launch_bounds__(NT) void k_line_lds(cx<T>* __restrict__ data, FftDe
     cx<T>* line = data + (long long)blockIdx.x * d.n;
     for (int e = threadIdx.x; e < d.n; e += NT) buf[e] = line[e];
     __syncthreads();
-    fft_lds<T, NT, MT>(buf, d, 1, tw, sgn);
+    fft_lds_either<T, NT, MT>(buf, d, 1, tw, sgn);
     for (int e = threadIdx.x; e < d.n; e += NT) line[e] = buf[e];
 }
 
@@ -65,10 +65,10 @@ __global__ __launch_bounds__(NT) void k_blue_lds(cx<T>* __restrict__ data, int N
     cx<T>* line = data + (long long)blockIdx.x * N;
     for (int e = threadIdx.x; e < dm.n; e += NT) buf[e] = e < N ? cmul(line[e], chirp[e]) : cx<T>{T(0), T(0)};
     __syncthreads();
-    fft_lds<T, NT, MT>(buf, dm, 1, tw, -1);
+    fft_lds<T, NT, MT, -1>(buf, dm, 1, tw);
     for (int e = threadIdx.x; e < dm.n; e += NT) buf[e] = cmul(buf[e], bhat[e]);
     __syncthreads();
-    fft_lds<T, NT, MT>(buf, dm, 1, tw, +1);
+    fft_lds<T, NT, MT, +1>(buf, dm, 1, tw);
     for (int e = threadIdx.x; e < N; e += NT) line[e] = cmul(buf[e], chirp[e]);
 }
 
@@ -90,7 +90,7 @@ __global__ __launch_bounds__(NT) void k_fs_cols(cx<T>* __restrict__ buf, int M1,
         s[c * M1 + a] = x[(long long)a * M2 + j0 + c];
     }
     __syncthreads();
-    fft_lds<T, NT, MT>(s, d1, nc, tw1, sgn);
+    fft_lds_either<T, NT, MT>(s, d1, nc, tw1, sgn);
     for (int e = threadIdx.x; e < nc * M1; e += NT) {
         const int a = e / nc, c = e - a * nc;
         cx<T> v = s[c * M1 + a];
@@ -113,7 +113,7 @@ __global__ __launch_bounds__(NT) void k_fs_rows(cx<T>* __restrict__ buf, int M1,
     cx<T>* x = buf + line * M + (long long)r0 * M2;
     for (int e = threadIdx.x; e < nr * M2; e += NT) s[e] = x[e];
     __syncthreads();
-    fft_lds<T, NT, MT>(s, d2, nr, tw2, sgn);
+    fft_lds_either<T, NT, MT>(s, d2, nr, tw2, sgn);
     for (int e = threadIdx.x; e < nr * M2; e += NT) {
         cx<T> v = s[e];
         if (twid) {

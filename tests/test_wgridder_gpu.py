@@ -388,6 +388,25 @@ def test_matrix_core_tiles_on_any_grid(nu, nv, single, supp):
     assert rel_linf(got, ref) < TOL_ORACLE[single]
 
 
+# single-precision plane lines that fill most of an LDS: their first pass reads
+# memory and their last one writes it; lengths that start with radix 3, 5, 8, 11
+# and 21 and end with 2, 4 and 8, up to the longest
+@pytest.mark.parametrize("long", [8232, 8250, 11264, 12100, 16384])
+@pytest.mark.parametrize("rows", [False, True])
+@pytest.mark.parametrize("wgridding", [True, False])
+def test_long_plane_lines(long, rows, wgridding, monkeypatch):
+    monkeypatch.setenv("RANG_FFT_TCM", "1")
+    supp = next(k for k, r in enumerate(W.kernel_table()) if r[0] == 5 and r[6] and r[1] < 1.7)
+    kernel = (supp, 64, long) if rows else (supp, long, 64)
+    uvw, freq, vis, wgt, nx, ny, dx = ref_case(nx=32, ny=30, field=0.3, wmax=400.0, nrow=60, seed=long)
+    got, ref, info, rinfo = v2d(uvw, freq, vis, wgt, nx, ny, dx, 1e-3, True, kernel=kernel, do_wgridding=wgridding)
+    same_plan(info, rinfo)
+    assert rel_linf(got, ref) < TOL_ORACLE[True]
+    x = np.random.default_rng(long).standard_normal((nx, ny))
+    got, ref, info, rinfo = d2v(uvw, freq, x, wgt, dx, 1e-3, True, kernel=kernel, do_wgridding=wgridding)
+    assert rel_linf(got, ref) < TOL_ORACLE[True]
+
+
 def test_double_batch_on_the_matrix_cores():
     # one launch per support, images of several supports in one batch
     import torch
