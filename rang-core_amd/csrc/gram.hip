@@ -645,9 +645,13 @@ struct GramImpl final : GramBase {
     // operator's first application, which sizes the slices).
     //
     // A column pass reading the n x 2n slice in place touches one cell per
-    // row; once a slice outgrows the caches (256 MiB and more, n >= 4096 in
-    // single precision) the slices are transposed through LDS tiles around
-    // the column pass instead, which then reads and writes whole columns
+    // row; the slices may be transposed through LDS tiles around the column
+    // pass instead, which then reads and writes whole columns. Applications of
+    // eight nodes, in place / transposed: single precision 1024^2 (16 MiB)
+    // 476 / 506 us, 1250^2 (24 MiB) 996 / 997, 1536^2 (36 MiB) 1780 / 1590,
+    // 2048^2 3393 / 3148, 2500^2 10.7 / 7.8 ms; double 1024^2 (32 MiB) 1260 /
+    // 1454 us, 2048^2 (128 MiB) 7.0 / 7.9 ms. So from 32 MiB in single and, once
+    // a slice outgrows the caches, 256 MiB in double precision
     // (RANG_GRAM_TRANSPOSE=0 or 1 forces either form, a test knob read with
     // the pass budget).
     int pass_nodes = 0;
@@ -657,7 +661,7 @@ struct GramImpl final : GramBase {
             if (e[0] == '0') return false;
             if (e[0] == '1') return true;
         }
-        return slice >= (std::size_t(256) << 20);
+        return slice >= (std::size_t(sizeof(T) == 4 ? 32 : 256) << 20);
     }
     int nodes_per_pass() const {
         std::size_t budget = std::size_t(2) << 30;
