@@ -271,7 +271,7 @@ __global__ __launch_bounds__(256, 2) void k_conv3_fwd(const std::uint16_t* __res
 // KS 3 (zero padding) or 1: a product over pixels.
 //
 // A workgroup takes 32 WCO output by 32 WCI input channels and runs over its
-// share of the tiles of 4 rows x 32 columns. A tile's dy and x (with the
+// share of the tiles of 8 rows x 32 columns. A tile's dy and x (with the
 // halo) are staged in LDS transposed, channel by channel along w: a thread
 // loads 8 pixels of 8 channels and turns the 8 x 8 block with 32 byte
 // permutes, so that 8 consecutive pixels of one channel are 16 contiguous
@@ -279,12 +279,16 @@ __global__ __launch_bounds__(256, 2) void k_conv3_fwd(const std::uint16_t* __res
 // pixel either way is formed from the row's registers and the two
 // neighbouring words by funnel shifts, not read again. A wave holds 32 x 32
 // channels of every tap (36 result tiles); where the channels do not occupy
-// the four waves, they split the tile's rows and are summed through LDS at
-// the end, one atomic add per weight and workgroup.
+// the eight waves, they split the tile's rows and are summed through LDS at
+// the end, one atomic add per weight and workgroup. One workgroup of eight
+// waves per CU, not two of four: the FP32 adds of the workgroups' sums are
+// most of the error, and half of them give 0.7 of it.
 // Measured (four 1024^2 images, four levels of 32 channels and up, 14
-// launches): 84.8 ms -> 4.4 ms; the kernel before it read its operands
+// launches): 84.8 ms -> 5.1 ms (4.4 as twice the workgroups, error against 64
+// bits of a 32- or 64-channel gradient 4.1e-7 and 2.9e-7 instead of 2.9e-7
+// and 2.1e-7); the kernel before it read its operands
 // two bytes at a time.
-constexpr int kWgRows = 4;
+constexpr int kWgRows = 8, kWgThreads = 512;
 template <int KS>
 struct WgradTile {
     static constexpr int halo = KS / 2;
@@ -316,12 +320,12 @@ __device__ __forceinline__ void store_turned(const uint4 (&v)[8], unsigned char*
 }
 
 template <int KS, int WCO, int WCI>
-__global__ __launch_bounds__(256, 2) void k_conv_wgrad(const std::uint16_t* __restrict__ x, int ldx, int xoff,
+__global__ __launch_bounds__(kWgThreads, 2) void k_conv_wgrad(const std::uint16_t* __restrict__ x, int ldx, int xoff,
                                                        const std::uint16_t* __restrict__ dy, int lddy, int dyoff,
                                                        float* __restrict__ dw, int H, int W, int cin, int cout,
                                                        int nth, int ntw, int ntiles, int nci, int xvec, int yvec) {
     using Tile = WgradTile<KS>;
-    constexpr int T = KS * KS, HALO = Tile::halo, WK = 4 / (WCO * WCI);
+    constexpr int T = KS * KS, HALO = Tile::halo, WK = kWgThreads / 64 / (WCO * WCI);
     constexpr int COB = 32 * WCO, CIB = 32 * WCI;
     extern __shared__ __align__(16) unsigned char wg_smem[];
     unsigned char* sx = wg_smem;
@@ -347,7 +351,7 @@ __global__ __launch_bounds__(256, 2) void k_conv_wgrad(const std::uint16_t* __re
         __syncthreads();  // the previous tile is consumed
         // blocks of 8 pixels x 8 channels: x rows with the halo, then dy rows
         constexpr int XB = Tile::xrows * 4 * (CIB / 8), YB = kWgRows * 4 * (COB / 8);
-        for (int e = tid; e < XB + YB; e += 256) {
+        for (int e = tid; e < XB + YB; e += kWgThreads) {
             const bool isx = e < XB;
             const int f = isx ? e : e - XB;
             const int no = isx ? CIB / 8 : COB / 8;
@@ -369,7 +373,7 @@ __global__ __launch_bounds__(256, 2) void k_conv_wgrad(const std::uint16_t* __re
         }
         if constexpr (HALO == 1) {
             // the columns w0 - 1 and w0 + 32
-            for (int e = tid; e < Tile::xrows * 2 * (CIB / 8); e += 256) {
+            for (int e = tid; e < Tile::xrows * 2 * (CIB / 8); e += kWgThreads) {
                 const int oct = e % (CIB / 8), g = e / (CIB / 8);
                 const int side = g & 1, r = g >> 1;
                 const int hh = h0 + r - 1, ww = side ? w0 + 32 : w0 - 1;
@@ -846,15 +850,15 @@ int32_t wgrad_launch(const std::uint16_t* x, int ldx, int xoff, const std::uint1
     const long long ntiles = (long long)B * nth * ntw;
     if (ntiles >= (1LL << 30)) return g_nn_err = "too many pixels for one weight gradient", 1;
     const int nco = (cout + 32 * WCO - 1) / (32 * WCO), nci = (cin + 32 * WCI - 1) / (32 * WCI);
-    // two workgroups per CU (their LDS), each with its share of the tiles
-    const long long want = (512 + nco * nci - 1) / (nco * nci);
+    // a workgroup per CU (its LDS), each with its share of the tiles
+    const long long want = (256 + nco * nci - 1) / (nco * nci);
     const unsigned nwg = unsigned(ntiles < want ? ntiles : want);
     const std::size_t lds = WgradTile<KS>::lds(32 * WCI, 32 * WCO);
     const auto kernel = k_conv_wgrad<KS, WCO, WCI>;
     if (const int e = nn_fail(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
                                                   hipFuncAttributeMaxDynamicSharedMemorySize, int(lds))))
         return e;
-    kernel<<<dim3(nwg, unsigned(nco * nci)), 256, lds, st>>>(x, ldx, xoff, dy, lddy, dyoff, dw, H, W, cin, cout, nth,
+    kernel<<<dim3(nwg, unsigned(nco * nci)), kWgThreads, lds, st>>>(x, ldx, xoff, dy, lddy, dyoff, dw, H, W, cin, cout, nth,
                                                             ntw, int(ntiles), nci, aligned16(x, ldx, xoff),
                                                             aligned16(dy, lddy, dyoff));
     return nn_fail(hipGetLastError());
