@@ -47,6 +47,7 @@
 #include "gram.h"
 #include "wg_device.h"
 #include "wg_fft.h"
+#include "wg_place.h"
 
 namespace rang {
 
@@ -377,11 +378,6 @@ struct Geo {
     int mfma;
 };
 
-// Width in u and v of a tile: the matrix-core gridding's last tiles may be
-// partial (every other tiling divides the grid).
-__device__ __forceinline__ int tile_wu(const Geo& g, int tu) { return min(g.Tu, g.nu - tu * g.Tu); }
-__device__ __forceinline__ int tile_wv(const Geo& g, int tv) { return min(g.Tv, g.nv - tv * g.Tv); }
-
 __device__ __forceinline__ int upos(const Geo& g, int u) { return g.lu1 ? (u % g.lu1) * g.lu2 + u / g.lu1 : u; }
 __device__ __forceinline__ int vpos(const Geo& g, int v) { return g.lv1 ? (v % g.lv1) * g.lv2 + v / g.lv1 : v; }
 
@@ -413,14 +409,6 @@ struct Rec {
 
 constexpr std::uint32_t kFlip = 0x80000000u;
 constexpr std::uint32_t kNoKey = 0xffffffffu;
-
-__device__ __forceinline__ void coord_of(const DevIn& in, const Geo& g, int row, double c[3]) {
-    const double tu = g.fu * in.uvw[3 * row], tv = g.fv * in.uvw[3 * row + 1];
-    const double tw = g.fw * in.uvw[3 * row + 2];
-    c[0] = tu + g.r_l * tw;
-    c[1] = tv + g.r_m * tw;
-    c[2] = tw;
-}
 
 __device__ __forceinline__ void sincos_t(float a, float& s, float& c) { sincosf(a, &s, &c); }
 __device__ __forceinline__ void sincos_t(double a, double& s, double& c) { sincos(a, &s, &c); }
@@ -478,31 +466,6 @@ __device__ __forceinline__ bool active(const DevIn& in, long long i) {
     return tnorm * twgt * tmask != 0.0;
 }
 
-// The first cell of a footprint and the position from it. u + ushift lies in
-// [nu - supp / 2, 2 nu + 1): 32-bit cells, one conditional step to wrap them.
-__device__ __forceinline__ void getpix(const Geo& g, double uin, double vin, double& uf,
-                                       double& vf, int& iu0, int& iv0) {
-    double u = uin * g.pixsize_x;
-    u = (u - floor(u)) * double(g.nu);
-    iu0 = min(int(u + g.ushift) - g.nu, int(g.maxiu0));
-    uf = u - double(iu0);
-    double v = vin * g.pixsize_y;
-    v = (v - floor(v)) * double(g.nv);
-    iv0 = min(int(v + g.vshift) - g.nv, int(g.maxiv0));
-    vf = v - double(iv0);
-}
-
-// (i0 + n / 2) mod n for i0 in [-n / 2, n + n / 2).
-__device__ __forceinline__ int shifted(int i0, int n) {
-    int v = i0 + n / 2;
-    if (v < 0) v += n;
-    return v >= n ? v - n : v;
-}
-
-// x / d with m = ceil(2^32 / d): exact for x d < 2^32 (grid sides below 2^20
-// times tiles of 8 to 64 cells).
-__device__ __forceinline__ int tile_of(int x, unsigned m) { return int(__umulhi(unsigned(x), m)); }
-
 // Row of sample i: the product with 1 / nchan is off by less than one unit in
 // the last place of a double, so its floor by at most one.
 __device__ __forceinline__ unsigned row_of(const Geo& g, unsigned i) {
@@ -511,13 +474,6 @@ __device__ __forceinline__ unsigned row_of(const Geo& g, unsigned i) {
     if (r * nchan > i) --r;
     if (i - r * nchan >= nchan) ++r;
     return r;
-}
-
-__device__ __forceinline__ int minplane(const Geo& g, double w) {
-    if (!g.wgrid) return 0;
-    const double p = (w + g.wshift) * g.xdw;
-    const int m = p > 0.0 ? int(min(p, 2147483647.0)) : 0;
-    return min(m, g.nb - 1);
 }
 
 // Shift phase of a visibility (wgridder.rs:1395-1408).
@@ -612,38 +568,12 @@ __global__ __launch_bounds__(256) void k_scan_final(const unsigned long long* bc
 
 // ------------------------------------------------------------ sort
 
-// Where a visibility falls on the grid: its FixW-signed coordinates, the
-// position of its footprint and its bucket (tile, spill class, first plane).
-// The spill class says whether its footprint reaches the next tile in u (2)
-// and in v (1).
-struct Place {
-    double imflip, b[3];  // the sign of w and the coordinates times it
-    double w, uf, vf;
-    int ou, ov, mp;
-    std::uint32_t key;
-};
-
+// Where a visibility falls on the grid, and its bucket. The count and the scatter
+// each place it (place_at rounds alike in both).
 __device__ __forceinline__ Place place_of(const DevIn& in, const Geo& g, unsigned row, unsigned ch) {
-    Place r;
     double c[3];
-    coord_of(in, g, int(row), c);
-    r.imflip = c[2] < 0.0 ? -1.0 : 1.0;  // FixW (wgridder.rs:583-586)
-    r.b[0] = c[0] * r.imflip;
-    r.b[1] = c[1] * r.imflip;
-    r.b[2] = c[2] * r.imflip;
-    const double f = in.foc[ch];
-    const double u = r.b[0] * f, v = r.b[1] * f;
-    r.w = r.b[2] * f;
-    int iu0, iv0;
-    getpix(g, u, v, r.uf, r.vf, iu0, iv0);
-    const int su = shifted(iu0, g.nu), sv = shifted(iv0, g.nv);
-    const int tu = tile_of(su, g.mTu), tv = tile_of(sv, g.mTv);
-    r.ou = su - tu * g.Tu;
-    r.ov = sv - tv * g.Tv;
-    const int cat = ((r.ou + g.supp > tile_wu(g, tu)) ? 2 : 0) | ((r.ov + g.supp > tile_wv(g, tv)) ? 1 : 0);
-    r.mp = minplane(g, r.w);
-    r.key = std::uint32_t((((long long)tu * g.ntv + tv) * 4 + cat) * g.nb + r.mp);
-    return r;
+    coord_of(g, in.uvw + 3 * row, c);
+    return place_at(g, c, in.foc[ch]);
 }
 
 // Runs of equal keys among the consecutive lanes of a wave (channels of one

@@ -282,3 +282,29 @@ def test_graph_replays_match_eager_calls(single):
         img, q = p.residual(v, x, out=d)
         img0, q0 = p.residual(v, x)
         assert rel_linf(host(img), host(img0)) < TOL[single] and abs(q - q0) <= 1e-12 * q0, k
+
+
+@pytest.mark.parametrize("single", [False, True])
+@pytest.mark.parametrize("spacing", [0.7, 5.3, 23.7])
+def test_prepared_with_visibilities_on_plane_boundaries(single, spacing):
+    """Evenly spaced w, one channel: the middle one lies on a plane boundary to
+    within a rounding; both record sets of the plan hold every visibility once."""
+    from rang.prepared import Prepared
+
+    nx, ny, dx = 48, 40, 0.2 / 48
+    freq = np.array([1.0e9])
+    k = np.arange(61)
+    rng = np.random.default_rng(61)
+    uvw = np.stack([rng.uniform(-0.4, 0.4, 61) / dx * 0.2998, rng.uniform(-0.4, 0.4, 61) / dx * 0.2998,
+                    np.where(k % 2, -1.0, 1.0) * k * spacing], axis=1)
+    cdt, rdt = (np.complex64, np.float32) if single else (np.complex128, np.float64)
+    vis = (rng.standard_normal((61, 1)) + 1j * rng.standard_normal((61, 1))).astype(cdt)
+    wgt = rng.uniform(0.5, 1.5, (61, 1)).astype(rdt)
+    eps = 1e-5 if single else 1e-9
+    p = Prepared(opts(nx, ny, dx, eps), dev(uvw), dev(freq), dev(wgt), single=single)
+    got = host(p.vis2dirty(dev(vis)))
+    assert rel_linf(got, oracle_image(uvw, freq, vis, wgt, nx, ny, dx, eps, single)) < TOL[single]
+    img = rng.standard_normal((nx, ny)).astype(rdt)
+    pv = host(p.dirty2vis(dev(img)))
+    assert rel_linf(pv, oracle_predict(uvw, freq, img, wgt, dx, eps)) < TOL[single]
+    p.close()

@@ -429,3 +429,37 @@ def test_double_batch_on_the_matrix_cores():
         # support 13 at oversampling 1.35: the correction at the image's edge
         # amplifies the sums' rounding by 1e5 (5e-11 with the LDS gridder too)
         assert rel_linf(d.cpu().numpy(), ref) < 1e-10
+
+
+def boundary_case(nu, nv, supp, spacing, K=40, nchan=1):
+    """Evenly spaced w from 0 (the middle one then often lies on a plane boundary
+    to within a rounding), u and v on the edges of cells, tiles among them."""
+    nx, ny, dx = 32, 30, 0.3 / 32
+    freq = np.linspace(1.0e9, 1.0e9 + 1e8 * (nchan - 1), nchan)
+    f = freq[0] / C_LIGHT
+    k = np.arange(K + 1)
+    half = 0.5 if supp % 2 else 0.0
+    uvw = np.stack([((k * 5) % nu - nu // 2 + half) / (nu * dx * f), ((k * 7) % nv - nv // 2 + half) / (nv * dx * f),
+                    np.where(k % 2, -1.0, 1.0) * k * spacing], axis=1)
+    rng = np.random.default_rng(K + supp)
+    vis = rng.standard_normal((K + 1, nchan)) + 1j * rng.standard_normal((K + 1, nchan))
+    return uvw, freq, vis, rng.uniform(0.5, 1.5, vis.shape), nx, ny, dx
+
+
+# visibilities within a rounding of the boundaries of planes, cells and tiles: the
+# sort's count and its scatter find one bucket, the oracle's
+@pytest.mark.parametrize("nu,nv", [(64, 66), (96, 80)])
+@pytest.mark.parametrize("single,supp", [(True, 4), (True, 7), (False, 5), (False, 8), (False, 13)])
+@pytest.mark.parametrize("nchan", [1, 3])
+def test_visibilities_on_bucket_boundaries(nu, nv, single, supp, nchan):
+    rows = [k for k, r in enumerate(W.kernel_table()) if r[0] == supp and (r[6] or not single) and r[1] < 1.7]
+    kernel = (rows[len(rows) // 2], nu, nv)
+    for spacing in (0.31, 1.7, 5.3, 11.9, 23.7, 41.1):
+        uvw, freq, vis, wgt, nx, ny, dx = boundary_case(nu, nv, supp, spacing, nchan=nchan)
+        got, ref, info, rinfo = v2d(uvw, freq, vis, wgt, nx, ny, dx, 1e-3, single, kernel=kernel)
+        same_plan(info, rinfo)
+        assert rel_linf(got, ref) < TOL_ORACLE[single]
+        x = np.random.default_rng(nv).standard_normal((nx, ny))
+        got, ref, info, rinfo = d2v(uvw, freq, x, wgt, dx, 1e-3, single, kernel=kernel)
+        same_plan(info, rinfo)
+        assert rel_linf(got, ref) < TOL_ORACLE[single]
