@@ -3162,15 +3162,7 @@ std::vector<double> table_key(const Geometry& G, const Geo& g) {
 // 0, where the visibility density peaks), densest first: a counting sort over
 // kRings rings on the GPU, in any order within a ring. (A sort on the host took
 // 17 ms for 446 x 446 tiles and an upload, at every change of the geometry.)
-constexpr int kRings = 1024;
 constexpr int kRingTiles = 4096;  // per block
-
-__device__ __forceinline__ int ring_of(const Geo& g, int t, float scale) {
-    const int tu = t / g.ntv, tv = t - tu * g.ntv;
-    const float cu = (float(tu) + 0.5f) * float(g.Tu) - 0.5f * float(g.nu);
-    const float cv = (float(tv) + 0.5f) * float(g.Tv) - 0.5f * float(g.nv);
-    return min(kRings - 1, int(sqrtf(cu * cu + cv * cv) * scale));
-}
 
 // Pass 0: the rings' counts. Pass 1, after k_ring_scan: each block takes its
 // places in every ring with one atomic and deals them out in LDS.

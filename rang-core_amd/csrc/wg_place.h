@@ -109,6 +109,19 @@ RANG_PLACE Place place_at(const Geo& g, const double c[3], double f) {
     return r;
 }
 
+// Ring of tile t: the distance of its centre from the grid's centre in steps of
+// 1 / scale cells. Counted in one kernel and dealt out in another, as above.
+constexpr int kRings = 1024;
+template <class Geo>
+RANG_PLACE int ring_of(const Geo& g, int t, float scale) {
+#pragma clang fp contract(off)
+    const int tu = t / g.ntv, tv = t - tu * g.ntv;
+    const float cu = (float(tu) + 0.5f) * float(g.Tu) - 0.5f * float(g.nu);
+    const float cv = (float(tv) + 0.5f) * float(g.Tv) - 0.5f * float(g.nv);
+    const int ring = int(sqrtf(cu * cu + cv * cv) * scale);
+    return ring < kRings - 1 ? ring : kRings - 1;
+}
+
 }  // namespace rang
 
 #undef RANG_PLACE

@@ -5,7 +5,7 @@
 // contraction mode of the device code and fused multiply-adds enabled.
 // Prints: calls, visibilities, differing buckets, calls without a permutation,
 // planes that differ from the unfused formula, visibilities within an ulp of a
-// plane boundary.
+// plane boundary, grids whose tiles do not fill their rings.
 
 #include <algorithm>
 #include <cmath>
@@ -46,10 +46,38 @@ __attribute__((noinline)) void place(const Geo& g, const double* uvw, double f, 
     }
 }
 
+// The tile order's two passes: one keeps the counts alone, the other the rings.
+__attribute__((noinline)) void ring_counts(const Geo& g, float scale, int* count) {
+    for (int t = 0; t < g.ntu * g.ntv; ++t) ++count[rang::ring_of(g, t, scale)];
+}
+
+__attribute__((noinline)) void rings_of(const Geo& g, float scale, int* ring) {
+    for (int t = 0; t < g.ntu * g.ntv; ++t) ring[t] = rang::ring_of(g, t, scale);
+}
+
+// Whether every ring's count is that of the tiles dealt to it, each the ring of
+// the unfused distance.
+bool rings_agree(const Geo& g) {
+    const double far = 0.5 * std::sqrt(double(g.nu + g.Tu) * double(g.nu + g.Tu) + double(g.nv + g.Tv) * double(g.nv + g.Tv));
+    const float scale = float(rang::kRings / far);
+    std::vector<int> count(rang::kRings, 0), ring(g.ntu * g.ntv);
+    ring_counts(g, scale, count.data());
+    rings_of(g, scale, ring.data());
+    for (int t = 0; t < g.ntu * g.ntv; ++t) {
+        --count[ring[t]];
+        volatile float hu = (float(t / g.ntv) + 0.5f) * float(g.Tu), hv = (float(t % g.ntv) + 0.5f) * float(g.Tv);
+        volatile float cu = hu - 0.5f * float(g.nu), cv = hv - 0.5f * float(g.nv);
+        volatile float uu = cu * cu, vv = cv * cv;
+        volatile float d2 = uu + vv;
+        if (std::min(int(std::sqrt(d2) * scale), rang::kRings - 1) != ring[t]) return false;
+    }
+    return std::all_of(count.begin(), count.end(), [](int c) { return c == 0; });
+}
+
 }  // namespace
 
 int main() {
-    long long calls = 0, vis = 0, differ = 0, broken = 0, off = 0, edge = 0;
+    long long calls = 0, vis = 0, differ = 0, broken = 0, off = 0, edge = 0, rings = 0;
     for (int trial = 0; trial < 4000; ++trial) {
         const int K = 2 * (8 + trial % 61);  // even: the middle w is (wmin + wmax) / 2
         const double epss[] = {1e-3, 1e-5, 1e-7, 1e-9};
@@ -109,9 +137,18 @@ int main() {
             if (std::floor(p * (1.0 + 4e-16)) != std::floor(p * (1.0 - 4e-16))) ++edge;
         }
         if (!ok) ++broken;
+        // tile sides 8 to 64 on grids up to 6000 cells
+        Geo r = g;
+        r.Tu = 8 + trial % 57;
+        r.Tv = 8 + (trial / 3) % 57;
+        r.ntu = 3 + trial % 90;
+        r.ntv = 2 + (trial / 7) % 90;
+        r.nu = r.ntu * r.Tu - trial % 5;
+        r.nv = r.ntv * r.Tv - trial % 3;
+        if (!rings_agree(r)) ++rings;
         ++calls;
         vis += n;
     }
-    std::printf("%lld %lld %lld %lld %lld %lld\n", calls, vis, differ, broken, off, edge);
+    std::printf("%lld %lld %lld %lld %lld %lld %lld\n", calls, vis, differ, broken, off, edge, rings);
     return 0;
 }

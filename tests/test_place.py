@@ -1,7 +1,8 @@
 """Placement of visibilities (rang-core_amd/csrc/wg_place.h) on the host: the
 count and the scatter of the sort must find the same bucket also where w, u or v
 lie within a rounding of a plane, cell or tile boundary, and the bucket is the
-one of the unfused formula (wgridder.rs:1003-1031)."""
+one of the unfused formula (wgridder.rs:1003-1031); the two passes of the tile
+order must find the same ring."""
 
 import shutil
 import subprocess
@@ -30,6 +31,7 @@ def test_both_placements_agree_on_boundaries(tmp_path):
                     "-ffp-contract=fast-honor-pragmas", f"-I{CSRC}", str(ROOT / "tests" / "place_check.cpp"),
                     str(CSRC / "wg_plan.cpp"), "-o", str(exe)], check=True)
     out = subprocess.run([str(exe)], check=True, capture_output=True, text=True).stdout
-    calls, vis, differ, broken, off, edge = map(int, out.split())
+    calls, vis, differ, broken, off, edge, rings = map(int, out.split())
     assert calls == 4000 and edge > 1000  # the boundaries are reached
     assert (differ, broken, off) == (0, 0, 0), out
+    assert rings == 0, out  # the tile order's two passes likewise
