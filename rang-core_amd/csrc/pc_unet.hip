@@ -104,13 +104,18 @@ __global__ __launch_bounds__(256) void k_conv1_fwd(const std::uint16_t* __restri
     }
 }
 
-// Eight consecutive BF16 values (16 bytes): one load when the tensor's base,
-// stride and offset are multiples of 16 bytes (vec16), two of 8 bytes
-// otherwise.
-__device__ __forceinline__ uint4 load8(const std::uint16_t* p, bool vec16) {
-    if (vec16) return *reinterpret_cast<const uint4*>(p);
-    const uint2 a = *reinterpret_cast<const uint2*>(p), b = *reinterpret_cast<const uint2*>(p + 4);
-    return make_uint4(a.x, a.y, b.x, b.y);
+// Eight consecutive BF16 values in accesses of `unit` values (8, 4 or 1, uniform:
+// unit_of), as the tensor's base, stride and offset allow.
+__device__ __forceinline__ uint4 load8(const std::uint16_t* p, int unit) {
+    if (unit == 8) return *reinterpret_cast<const uint4*>(p);
+    if (unit == 4) {
+        const uint2 a = *reinterpret_cast<const uint2*>(p), b = *reinterpret_cast<const uint2*>(p + 4);
+        return make_uint4(a.x, a.y, b.x, b.y);
+    }
+    std::uint32_t r[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) r[k] = p[2 * k] | (std::uint32_t(p[2 * k + 1]) << 16);
+    return make_uint4(r[0], r[1], r[2], r[3]);
 }
 
 __device__ __forceinline__ bf16x8 as_bf16x8(uint4 v) { return __builtin_bit_cast(bf16x8, v); }
@@ -189,7 +194,7 @@ template <int WCO>
 __global__ __launch_bounds__(256, 2) void k_conv3_fwd(const std::uint16_t* __restrict__ x, int ldx, int xoff,
                                                       const std::uint16_t* __restrict__ w, float* __restrict__ y,
                                                       std::uint16_t* __restrict__ a, int ldy, int yoff, int H, int W,
-                                                      int cin, int cout, int relu, int nth, int ntw, int vec16,
+                                                      int cin, int cout, int relu, int nth, int ntw, int unit,
                                                       int out16) {
     using Tile = Conv3Tile<WCO>;
     constexpr int CO = Tile::co, HC = kConvCols + 2;
@@ -218,7 +223,7 @@ __global__ __launch_bounds__(256, 2) void k_conv3_fwd(const std::uint16_t* __res
             const int hh = h0 - 1 + px / HC, ww = w0 - 1 + px % HC;
             uint4 v = make_uint4(0u, 0u, 0u, 0u);
             if (oct < noct && hh >= 0 && hh < H && ww >= 0 && ww < W)
-                v = load8(xi + ((long long)hh * W + ww) * ldx + c0 + 8 * oct, vec16);
+                v = load8(xi + ((long long)hh * W + ww) * ldx + c0 + 8 * oct, unit);
             sx[px * kConvPixel + oct] = v;
         }
         const int per = 9 * noct;  // octets of one output channel
@@ -226,7 +231,7 @@ __global__ __launch_bounds__(256, 2) void k_conv3_fwd(const std::uint16_t* __res
             const int co = e / per, t = e - co * per;  // t = tap noct + octet
             const int tap = t / noct, oct = t - tap * noct;
             uint4 v = make_uint4(0u, 0u, 0u, 0u);
-            if (co0 + co < cout) v = load8(w + ((long long)(co0 + co) * 9 + tap) * cin + c0 + 8 * oct, vec16);
+            if (co0 + co < cout) v = load8(w + ((long long)(co0 + co) * 9 + tap) * cin + c0 + 8 * oct, unit);
             sw[t * CO + co] = v;
         }
         __syncthreads();
@@ -323,7 +328,7 @@ template <int KS, int WCO, int WCI>
 __global__ __launch_bounds__(kWgThreads, 2) void k_conv_wgrad(const std::uint16_t* __restrict__ x, int ldx, int xoff,
                                                        const std::uint16_t* __restrict__ dy, int lddy, int dyoff,
                                                        float* __restrict__ dw, int H, int W, int cin, int cout,
-                                                       int nth, int ntw, int ntiles, int nci, int xvec, int yvec) {
+                                                       int nth, int ntw, int ntiles, int nci, int xunit, int yunit) {
     using Tile = WgradTile<KS>;
     constexpr int T = KS * KS, HALO = Tile::halo, WK = kWgThreads / 64 / (WCO * WCI);
     constexpr int COB = 32 * WCO, CIB = 32 * WCI;
@@ -361,11 +366,11 @@ __global__ __launch_bounds__(kWgThreads, 2) void k_conv_wgrad(const std::uint16_
             const int ld = isx ? ldx : lddy;
             const bool live = hh >= 0 && hh < H && (isx ? cib + 8 * oct < cin : cob + 8 * oct < cout);
             const std::uint16_t* src = (isx ? xi : yi) + ((long long)hh * W + w0 + 8 * j) * ld + 8 * oct;
-            const bool vec = isx ? xvec : yvec;
+            const int unit = isx ? xunit : yunit;
             uint4 v[8];
 #pragma unroll
             for (int p = 0; p < 8; ++p)
-                v[p] = live && w0 + 8 * j + p < W ? load8(src + (long long)p * ld, vec) : zero;
+                v[p] = live && w0 + 8 * j + p < W ? load8(src + (long long)p * ld, unit) : zero;
             if (isx)
                 store_turned(v, sx + 8 * oct * Tile::xstride + r * 96 + 16 + 16 * j, Tile::xstride);
             else
@@ -379,7 +384,7 @@ __global__ __launch_bounds__(kWgThreads, 2) void k_conv_wgrad(const std::uint16_
                 const int hh = h0 + r - 1, ww = side ? w0 + 32 : w0 - 1;
                 uint4 v = zero;
                 if (hh >= 0 && hh < H && ww >= 0 && ww < W && cib + 8 * oct < cin)
-                    v = load8(xi + ((long long)hh * W + ww) * ldx + 8 * oct, xvec);
+                    v = load8(xi + ((long long)hh * W + ww) * ldx + 8 * oct, xunit);
                 const std::uint32_t d[4] = {v.x, v.y, v.z, v.w};
                 unsigned char* at = sx + 8 * oct * Tile::xstride + r * 96 + (side ? 80 : 14);
 #pragma unroll
@@ -815,8 +820,13 @@ int grid1(long long n) {
     return int(b < 1 ? 1 : b > 65536 ? 65536 : b);
 }
 
-bool aligned16(const void* p, int ld, int off) {
-    return reinterpret_cast<std::uintptr_t>(p) % 16 == 0 && ld % 8 == 0 && off % 8 == 0;
+// Values per access of load8 for a BF16 tensor: 16 or 8 bytes where its base,
+// stride and offset are multiples of them, else one value.
+int unit_of(const void* p, int ld, int off) {
+    const std::uintptr_t at = reinterpret_cast<std::uintptr_t>(p);
+    if (at % 16 == 0 && ld % 8 == 0 && off % 8 == 0) return 8;
+    if (at % 8 == 0 && ld % 4 == 0 && off % 4 == 0) return 4;
+    return 1;
 }
 
 // Whether 8 channels from a multiple of 8 can be read in 16-byte accesses.
@@ -828,7 +838,7 @@ bool vector8(const E* p, int ld, int off) {
 
 template <int WCO>
 int32_t conv3_launch(const std::uint16_t* x, int ldx, int xoff, const std::uint16_t* w, float* y, std::uint16_t* a, int ldy,
-                            int yoff, int B, int H, int W, int cin, int cout, int relu, int vec16, int out16,
+                            int yoff, int B, int H, int W, int cin, int cout, int relu, int unit, int out16,
                             hipStream_t st) {
     using Tile = Conv3Tile<WCO>;
     const int nth = (H + Tile::rows - 1) / Tile::rows, ntw = (W + kConvCols - 1) / kConvCols;
@@ -839,7 +849,7 @@ int32_t conv3_launch(const std::uint16_t* x, int ldx, int xoff, const std::uint1
                                                   hipFuncAttributeMaxDynamicSharedMemorySize, int(Tile::lds))))
         return e;
     kernel<<<dim3(unsigned(blocks), unsigned((cout + Tile::co - 1) / Tile::co)), 256, Tile::lds, st>>>(
-        x, ldx, xoff, w, y, a, ldy, yoff, H, W, cin, cout, relu, nth, ntw, vec16, out16);
+        x, ldx, xoff, w, y, a, ldy, yoff, H, W, cin, cout, relu, nth, ntw, unit, out16);
     return nn_fail(hipGetLastError());
 }
 
@@ -859,8 +869,8 @@ int32_t wgrad_launch(const std::uint16_t* x, int ldx, int xoff, const std::uint1
                                                   hipFuncAttributeMaxDynamicSharedMemorySize, int(lds))))
         return e;
     kernel<<<dim3(nwg, unsigned(nco * nci)), kWgThreads, lds, st>>>(x, ldx, xoff, dy, lddy, dyoff, dw, H, W, cin, cout, nth,
-                                                            ntw, int(ntiles), nci, aligned16(x, ldx, xoff),
-                                                            aligned16(dy, lddy, dyoff));
+                                                            ntw, int(ntiles), nci, unit_of(x, ldx, xoff),
+                                                            unit_of(dy, lddy, dyoff));
     return nn_fail(hipGetLastError());
 }
 
@@ -899,14 +909,14 @@ int32_t rang_amd_nn_conv_fwd(const uint16_t* x, int32_t ldx, int32_t xoff, const
         k_conv1_fwd<<<grid, 256, 0, st>>>(x, ldx, xoff, w, y, a, ldy, yoff, npix, cin, cout, relu);
         return nn_fail(hipGetLastError());
     }
-    const int vec16 = aligned16(x, ldx, xoff) && aligned16(w, 8, 0);
+    const int ux = unit_of(x, ldx, xoff), uw = unit_of(w, 8, 0), unit = ux < uw ? ux : uw;
     const int out16 = ldy % 4 == 0 && yoff % 4 == 0 && reinterpret_cast<uintptr_t>(y) % 16 == 0 &&
                       reinterpret_cast<uintptr_t>(a) % 8 == 0;
     // 64 output channels a workgroup where they divide evenly: half the
     // reads of the input
     if (cout % 64 == 0)
-        return conv3_launch<2>(x, ldx, xoff, w, y, a, ldy, yoff, B, H, W, cin, cout, relu, vec16, out16, st);
-    return conv3_launch<1>(x, ldx, xoff, w, y, a, ldy, yoff, B, H, W, cin, cout, relu, vec16, out16, st);
+        return conv3_launch<2>(x, ldx, xoff, w, y, a, ldy, yoff, B, H, W, cin, cout, relu, unit, out16, st);
+    return conv3_launch<1>(x, ldx, xoff, w, y, a, ldy, yoff, B, H, W, cin, cout, relu, unit, out16, st);
 }
 
 int32_t rang_amd_nn_conv_wgrad(const uint16_t* x, int32_t ldx, int32_t xoff, const uint16_t* dy, int32_t lddy,

@@ -130,6 +130,46 @@ def test_conv3_tile_edges(cin, cout, H, W, pad):
     assert float((torch_weight(dw.cpu(), 3).double() - ref_dw).abs().max()) <= bound
 
 
+# output gradients at any stride, offset and base (one value an access where
+# neither 16 nor 8 bytes are aligned), and inputs at any base
+@pytest.mark.parametrize("ks", [1, 3])
+@pytest.mark.parametrize("pad,off,xshift,yshift", [(1, 1, 0, 0), (2, 2, 0, 0), (6, 2, 0, 0), (4, 4, 0, 1), (0, 0, 1, 3),
+                                                   (0, 0, 4, 4), (0, 0, 2, 0)])
+def test_weight_gradient_at_any_alignment(ks, pad, off, xshift, yshift):
+    from rang import precond as P
+
+    lib, st = P._lib(), P._stream()
+    g = torch.Generator().manual_seed(100 * ks + 10 * pad + xshift + yshift)
+    B, H, W, cin, cout = 2, 9, 33, 48, 32
+    n, ld = B * H * W, cout + pad
+    xb = torch.zeros(n * cin + 8, dtype=torch.int16, device="cuda")
+    yb = torch.zeros(n * ld + 8, dtype=torch.int16, device="cuda")
+    x, dy = torch.randn(n, cin, generator=g), torch.randn(n, ld, generator=g)
+    xb[xshift:xshift + n * cin] = bf16_bits(x).cuda().reshape(-1)
+    yb[yshift:yshift + n * ld] = bf16_bits(dy).cuda().reshape(-1)
+    dw = torch.zeros(cout, ks * ks, cin, device="cuda")
+    P._ok(lib.rang_amd_nn_conv_wgrad(P._p(xb[xshift:]), cin, 0, P._p(yb[yshift:]), ld, off, P._p(dw), B, H, W, cin, cout,
+                                     ks, st))
+    xr = nchw(from_bits(bf16_bits(x)), B, H, W, cin).double()
+    dyr = nchw(from_bits(bf16_bits(dy))[:, off:off + cout].contiguous(), B, H, W, cout).double()
+    shape = (cout, cin, ks, ks)
+    ref = torch.nn.grad.conv2d_weight(xr, shape, dyr, padding=ks // 2)
+    # FP32 sums of n exact products: each addition rounds by 2^-24 of the sum of magnitudes
+    bound = n * 2.0 ** -24 * float(torch.nn.grad.conv2d_weight(xr.abs(), shape, dyr.abs(), padding=ks // 2).max())
+    assert float((torch_weight(dw.cpu(), ks).double() - ref).abs().max()) <= bound
+    # the forward product from the same base
+    w = torch.randn(cout, ks * ks, cin, generator=g) / math.sqrt(ks * ks * cin)
+    wb = bf16_bits(w).cuda()
+    if ks == 3:
+        y = torch.zeros(n, cout, device="cuda")
+        P._ok(lib.rang_amd_nn_conv_fwd(P._p(xb[xshift:]), cin, 0, P._p(wb), P._p(y), None, cout, 0, B, H, W, cin, cout,
+                                       ks, 0, st))
+        wr = torch_weight(from_bits(bf16_bits(w)), ks).double()
+        ref = F.conv2d(xr, wr, padding=1)
+        bound = 9 * cin * 2.0 ** -24 * float(F.conv2d(xr.abs(), wr.abs(), padding=1).max())
+        assert float((nchw(y.cpu(), B, H, W, cout).double() - ref).abs().max()) <= bound
+
+
 # eight channels a thread (16, 0), or one where the stride (pad 2) or the channel
 # count does not allow it
 @pytest.mark.parametrize("C,pad", [(16, 0), (24, 8), (16, 2), (12, 0)])
