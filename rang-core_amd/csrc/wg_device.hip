@@ -374,9 +374,11 @@ struct Geo {
     // Transforms longer than one LDS along u or v: n = n1 n2 (0: in LDS).
     // Their forward results sit at (k mod n1) n2 + k / n1.
     int lu1, lu2, lv1, lv2;
-    // Gridding on the matrix cores (16 x 16 tiles, k_grid_mfma).
+    // Gridding on the matrix cores (grid_item_mfma; 0: in LDS) and the type its
+    // sums are held in.
     int mfma;
 };
+constexpr int kMfmaSingle = 1, kMfmaDouble = 2;
 
 __device__ __forceinline__ int upos(const Geo& g, int u) { return g.lu1 ? (u % g.lu1) * g.lu2 + u / g.lu1 : u; }
 __device__ __forceinline__ int vpos(const Geo& g, int v) { return g.lv1 ? (v % g.lv1) * g.lv2 + v / g.lv1 : v; }
@@ -871,15 +873,18 @@ __device__ __forceinline__ void source_range(const Geo& g, const std::uint32_t* 
     b = off[k0 + mhi + 1];
 }
 
+// With `split` the units of at most kShortItem records are counted apart, after
+// the others (2 ntg counts).
+constexpr std::uint32_t kShortItem = 64;
 __global__ __launch_bounds__(256) void k_grid_items(Geo g, const std::uint32_t* __restrict__ off,
                                                     const std::uint32_t* __restrict__ order, int G,
-                                                    int ngroups, int S, std::uint32_t rc,
+                                                    int ngroups, int S, std::uint32_t rc, int split,
                                                     std::uint32_t* __restrict__ nitems) {
     const int ntg = g.ntu * g.ntv * ngroups;
     const int tg = blockIdx.x * blockDim.x + threadIdx.x;
     if (tg > ntg) return;
     if (tg == ntg) {
-        nitems[ntg] = 0;
+        nitems[split ? 2 * ntg : ntg] = 0;
         return;
     }
     const int rank = tg / ngroups, grp = tg - rank * ngroups;
@@ -895,7 +900,17 @@ __global__ __launch_bounds__(256) void k_grid_items(Geo g, const std::uint32_t* 
         total += b - a;
     }
     // a unit without visibilities takes no item: k_zero_split clears its cells
-    nitems[tg] = (total + rc - 1) / rc;
+    const std::uint32_t n = (total + rc - 1) / rc;
+    const bool apart = split && total <= kShortItem;
+    nitems[tg] = apart ? 0 : n;
+    if (split) nitems[ntg + tg] = apart ? n : 0;
+}
+
+// Items of a unit from the prefix sums of those counts.
+__device__ __forceinline__ std::uint32_t items_of(const std::uint32_t* item_off, int ntg, int tg, int split) {
+    std::uint32_t n = item_off[tg + 1] - item_off[tg];
+    if (split) n += item_off[ntg + tg + 1] - item_off[ntg + tg];
+    return n;
 }
 
 // Cells of the (tile, plane group)s gridded by more than one item, zeroed
@@ -904,9 +919,10 @@ __global__ __launch_bounds__(256) void k_grid_items(Geo g, const std::uint32_t* 
 template <class T, int NOUT>
 __global__ __launch_bounds__(256) void k_zero_split(Geo g, const std::uint32_t* __restrict__ item_off,
                                                     const std::uint32_t* __restrict__ order, int G,
-                                                    int ngroups, cx<T>* __restrict__ grid, int skip_empty) {
+                                                    int ngroups, cx<T>* __restrict__ grid, int skip_empty,
+                                                    int split) {
     const int tg = blockIdx.x;
-    const std::uint32_t n = item_off[tg + 1] - item_off[tg];
+    const std::uint32_t n = items_of(item_off, int(gridDim.x), tg, split);
     if (n == 1 || (n == 0 && skip_empty)) return;
     const int rank = tg / ngroups, grp = tg - rank * ngroups;
     const int tile = int(order[rank]);
@@ -935,11 +951,11 @@ __global__ __launch_bounds__(256) void k_zero_split(Geo g, const std::uint32_t* 
 // occ[group][tile] = 1 when a gridding item reaches the (tile, plane group).
 __global__ __launch_bounds__(256) void k_occupancy(const std::uint32_t* __restrict__ item_off,
                                                    const std::uint32_t* __restrict__ order, int ntg, int ngroups,
-                                                   int ntiles, std::uint8_t* __restrict__ occ) {
+                                                   int ntiles, int split, std::uint8_t* __restrict__ occ) {
     const int tg = blockIdx.x * 256 + threadIdx.x;
     if (tg >= ntg) return;
     const int rank = tg / ngroups, grp = tg - rank * ngroups;
-    occ[(long long)grp * ntiles + order[rank]] = item_off[tg + 1] > item_off[tg] ? 1 : 0;
+    occ[(long long)grp * ntiles + order[rank]] = items_of(item_off, ntg, tg, split) ? 1 : 0;
 }
 
 // The item `item` of a prefix array of per-unit item counts: the unit and
@@ -974,9 +990,9 @@ constexpr int kGridBatch = 512;  // records staged in LDS at a time
 // visibilities share a position (the channels and times of a short baseline
 // do). NOUT = 2 grids a dirty image and a PSF together
 // (wgridder.rs:2128-2152). Row stride TvP is padded so that the S x S
-// footprint spreads over the banks. The accumulators are double in both
-// precisions: LDS adds of doubles run some twenty times faster than those of
-// floats on CDNA4, and the sums only gain accuracy.
+// footprint spreads over the banks. This gridder's accumulators are double in
+// both precisions: LDS adds of doubles run some twenty times faster than those
+// of floats on CDNA4, and the sums only gain accuracy.
 using GridAcc = double;
 
 // Record j of an item's concatenated source ranges, with its in-tile offsets
@@ -1380,10 +1396,10 @@ __global__ __launch_bounds__(grid_threads<T>()) void k_grid_jobs(const GridJob<T
 
 // ------------------------------------------------------------ gridding on the matrix cores
 
-// W-gridding on 16 x 16 windows with the matrix cores: one wave per item
-// (tile, group of planes, chunk), whose accumulators are the item's planes of
-// the tile held in the MFMA result registers, so that no LDS atomics are
-// needed. Four visibilities at a time: with A[i][k] = ku_k(i - ou_k) kw_k(plane)
+// W-gridding on 16 x 16 windows with the matrix cores: an item (tile, group of
+// planes, chunk) is one wave's, or shared by several in single precision, and its
+// planes of the tile are held in the MFMA result registers, so that no LDS
+// atomics are needed per tap. Four visibilities at a time: with A[i][k] = ku_k(i - ou_k) kw_k(plane)
 // (lane 16 k + i) and B[k][j] = kv_k(j - ov_k) v_k (lane 16 k + j), one
 // v_mfma_f32_16x16x4_f32 or v_mfma_f64_16x16x4_f64 per plane and part adds
 // sum_k A[i][k] B[k][j] to cell (i, j) of the plane, which is the gridding sum
@@ -1401,6 +1417,20 @@ __global__ __launch_bounds__(grid_threads<T>()) void k_grid_jobs(const GridJob<T
 // dirty and PSF, support 7 (7 planes): the call 43.9 -> 17.4 ms, eight planes
 // an item at one wave per SIMD (256 registers of accumulators); four planes at
 // two waves 19.1, five 20.2. Support 11, 118 k visibilities: 720 -> 195 us.
+//
+// The LDS gridder forms products and sums in double in both precisions. Here
+// single-precision sums of one output on grids that tile by 16 stay in single
+// precision over an item (kMfmaSingle). Two outputs, and grids of other sides,
+// take double sums (kMfmaDouble): the registers hold the products of 64 records at
+// most and are then added to sums in LDS, for which their waves have 24 to 32 KiB
+// and a third of the LDS's add rate. Rounding error of an image (2-norm against
+// double precision with the same kernel), LDS gridder / single-precision sums of
+// up to 4096 records / these: dirty and PSF of 19.4 M visibilities, support 7,
+// 1.9e-7 / 5.3e-7 / 1.2e-7; 118 k visibilities on a few tiles 1.4e-6 / 3.2e-6 /
+// 1.1e-6; spread thinly over a grid 1.25 times the image (epsilon 1e-2), the least
+// favourable, 7.7e-7 / 1.0e-6 / 8.6e-7. Calls: 3.2 M visibilities, support 7, one
+// output 2.16 / 1.33 / 1.36 ms; support 6 thinly spread 2.08 / 1.14 / 1.21 ms; dirty and
+// PSF of 19.4 M 21.1 / 7.5 / 7.9 ms. On the f64 matrix cores: 2.04 ms for the first.
 constexpr int kMfmaPlanes = 8;
 
 // Lane q of each row of 16 lanes, broadcast to its row (DPP row_newbcast;
@@ -1448,14 +1478,31 @@ struct Mfma<double> {
     static __device__ __forceinline__ int row(int k, int r) { return k + 4 * r; }
 };
 
-template <class T, int S, int NOUT>
-struct MfmaShared {
-    T coef[2 * ne_of<S>() * S];
-    std::uint32_t start[9], pre[10];
+// A wave's LDS, after the item's sums where several waves share it.
+template <class T, int NOUT>
+struct alignas(16) MfmaWave {
     Rec<T> rec[64];
     cx<T> unit[NOUT == 2 ? 64 : 1];  // the second output's values
     int qr[32];  // per group of 4 staged records: its planes [lo, hi) in the item
+    std::uint32_t start[9], pre[10];
 };
+// Real and imaginary parts held per cell; the second output's imaginary part is
+// zero without shifts.
+__host__ __device__ inline int mfma_parts(const Geo& g, int nout) { return nout == 1 ? 2 : g.shifting ? 4 : 3; }
+__host__ __device__ inline std::size_t mfma_sums(const Geo& g, int nout, int G, int waves) {
+    return waves > 1 ? sizeof(double) * 256 * std::size_t(mfma_parts(g, nout)) * std::size_t(G) : 0;
+}
+template <class T, int NOUT>
+std::size_t mfma_lds(const Geo& g, int G, int waves) {
+    return mfma_sums(g, NOUT, G, waves) + sizeof(MfmaWave<T, NOUT>) * std::size_t(waves);
+}
+
+// Orders a wave's LDS writes before its other lanes' reads.
+__device__ __forceinline__ void wave_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
 
 template <class T, int S, int NOUT, bool FORM>
 __device__ __forceinline__ void grid_item_mfma(Geo g, const Rec<T>* __restrict__ recs,
@@ -1464,22 +1511,34 @@ __device__ __forceinline__ void grid_item_mfma(Geo g, const Rec<T>* __restrict__
                                                std::uint32_t rc, const std::uint32_t* __restrict__ item_off,
                                                const std::uint32_t* __restrict__ order,
                                                cx<T>* __restrict__ grid, std::uint32_t item, T* coef,
-                                               std::uint32_t* s_start, std::uint32_t* s_pre, Rec<T>* s_rec,
-                                               cx<T>* s_unit, int* s_qr) {
+                                               unsigned char* dyn_lds) {
     using M = Mfma<T>;
     using Acc = typename M::Acc;
     constexpr int NE = ne_of<S>(), KP = kMfmaPlanes;
-    const int lane = threadIdx.x;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int nwaves = int(blockDim.x) >> 6;
+    double* sums = reinterpret_cast<double*>(dyn_lds);
+    MfmaWave<T, NOUT>& sw = reinterpret_cast<MfmaWave<T, NOUT>*>(dyn_lds + mfma_sums(g, NOUT, G, nwaves))[wave];
+    Rec<T>* s_rec = sw.rec;
+    cx<T>* s_unit = sw.unit;
+    int* s_qr = sw.qr;
+    std::uint32_t* s_start = sw.start;
+    std::uint32_t* s_pre = sw.pre;
+    for (int e = tid; e < 2 * NE * S; e += int(blockDim.x)) coef[e] = coeff[e];
+    __syncthreads();
+    // several waves share a long item; short ones, which follow, take one each
     const int ntg = g.ntu * g.ntv * ngroups;
+    const bool split = sizeof(T) == 4 && nwaves > 1;
+    const bool lone = split && item >= item_off[ntg];
+    if (lone) item = item_off[ntg] + (item - item_off[ntg]) * unsigned(nwaves) + unsigned(wave);
     int tg;
     std::uint32_t chunk, nchunks;
-    if (!find_item(item_off, ntg, item, tg, chunk, nchunks)) return;
+    if (!find_item(item_off + (lone ? ntg : 0), ntg, item, tg, chunk, nchunks)) return;
     const int rank = tg / ngroups, grp = tg - rank * ngroups;
     const int tile = int(order[rank]);
     const int tu = tile / g.ntv, tv = tile - tu * g.ntv;
     const int P = g.nplanes;
     const int p0 = grp * G, p1 = min(P, p0 + G), np = p1 - p0;
-    for (int e = lane; e < 2 * NE * S; e += 64) coef[e] = coeff[e];
     const int mlo = max(0, p0 - S + 1), mhi = min(g.nb - 1, p1 - 1);
     if (lane < 9) {
         std::uint32_t a, b;
@@ -1487,12 +1546,12 @@ __device__ __forceinline__ void grid_item_mfma(Geo g, const Rec<T>* __restrict__
         s_start[lane] = a;
         s_pre[lane + 1] = b - a;
     }
-    __syncthreads();
+    wave_sync();
     if (lane == 0) {
         s_pre[0] = 0;
         for (int k = 1; k <= 9; ++k) s_pre[k] += s_pre[k - 1];
     }
-    __syncthreads();
+    wave_sync();
     const std::uint32_t jbeg = chunk * rc, jend = min(s_pre[9], jbeg + rc);
     const int k = lane >> 4, i = lane & 15;
     // up to support 8, lane 16 k + i holds tap i (u and w) for i < S and tap
@@ -1512,7 +1571,16 @@ __device__ __forceinline__ void grid_item_mfma(Geo g, const Rec<T>* __restrict__
         for (int q = 0; q < KP; ++q) are[o][q] = aim[o][q] = Acc{T(0), T(0), T(0), T(0)};
     // the second output's imaginary part is zero without shifts
     const bool unit_im = NOUT == 2 && g.shifting;
-    for (std::uint32_t base = jbeg; base < jend; base += 64) {
+    // several waves: their sums meet in LDS, after every batch or once each
+    const bool shared = split && !lone, fold = g.mfma == kMfmaDouble;
+    const std::uint32_t first = shared ? 64u * unsigned(wave) : 0u, step = shared ? 64u * unsigned(nwaves) : 64u;
+    if constexpr (sizeof(T) == 4) {
+        if (shared) {
+            for (int e = tid; e < mfma_parts(g, NOUT) * np * 256; e += int(blockDim.x)) sums[e] = 0.0;
+            __syncthreads();
+        }
+    }
+    for (std::uint32_t base = jbeg + first; base < jend; base += step) {
         const int nrec = int(min(jend - base, 64u));
         Rec<T> r{};
         cx<T> unit{T(0), T(0)};
@@ -1540,7 +1608,7 @@ __device__ __forceinline__ void grid_item_mfma(Geo g, const Rec<T>* __restrict__
             qb = max(qb, __shfl_xor(qb, 1, 64));
             qa = min(qa, __shfl_xor(qa, 2, 64));
             qb = max(qb, __shfl_xor(qb, 2, 64));
-            __syncthreads();  // the previous batch is consumed
+            wave_sync();  // the previous batch is consumed
             s_rec[lane] = r;
             if constexpr (NOUT == 2) s_unit[lane] = unit;
             if ((lane & 3) == 0) {
@@ -1548,7 +1616,7 @@ __device__ __forceinline__ void grid_item_mfma(Geo g, const Rec<T>* __restrict__
                 s_qr[(lane >> 1) + 1] = min(qb, np);
             }
         }
-        __syncthreads();
+        wave_sync();
         for (int g4 = 0; g4 < nrec; g4 += 4) {
             const Rec<T>& rk = s_rec[g4 + k];
             const std::uint32_t pos = rk.pos;
@@ -1612,10 +1680,56 @@ __device__ __forceinline__ void grid_item_mfma(Geo g, const Rec<T>* __restrict__
                 }
             }
         }
+        if constexpr (sizeof(T) == 4) {
+            if (shared && (fold || base + step >= jend)) {
+#pragma unroll
+                for (int o = 0; o < NOUT; ++o)
+#pragma unroll
+                    for (int q = 0; q < KP; ++q) {
+                        if (q >= np) break;
+                        double* at = sums + (2 * o * np + q) * 256 + lane;
+#pragma unroll
+                        for (int r4 = 0; r4 < 4; ++r4) atomicAdd(at + 64 * r4, double(are[o][q][r4]));
+                        are[o][q] = Acc{T(0), T(0), T(0), T(0)};
+                        if (o == 0 || unit_im) {
+#pragma unroll
+                            for (int r4 = 0; r4 < 4; ++r4)
+                                atomicAdd(at + np * 256 + 64 * r4, double(aim[o][q][r4]));
+                            aim[o][q] = Acc{T(0), T(0), T(0), T(0)};
+                        }
+                    }
+            }
+        }
+    }
+    const long long plane = (long long)g.nu * g.nv;
+    if constexpr (sizeof(T) == 4) {
+        if (shared) {
+            // each thread keeps a column, as its lane does below
+            __syncthreads();
+            if (i >= wv) return;
+            int gcol = tv * g.Tv + i + g.nv / 2;
+            if (gcol >= g.nv) gcol -= g.nv;
+            for (int e = wave; e < NOUT * np * 4; e += nwaves) {
+                const int o = e / (np * 4), f = e - o * np * 4, q = f >> 2, r4 = f & 3;
+                const int ti = M::row(k, r4);
+                if (ti >= wu) continue;
+                int grow = tu * g.Tu + ti + g.nu / 2;
+                if (grow >= g.nu) grow -= g.nu;
+                const double* at = sums + (2 * o * np + q) * 256 + 64 * r4 + lane;
+                const T vre = T(at[0]), vim = o == 0 || unit_im ? T(at[np * 256]) : T(0);
+                cx<T>* c = grid + ((long long)o * P + p0 + q) * plane + (long long)grow * g.nv + gcol;
+                if (nchunks == 1) {
+                    *c = cx<T>{vre, vim};
+                } else if (vre != T(0) || vim != T(0)) {
+                    atomicAdd(&c->re, vre);
+                    atomicAdd(&c->im, vim);
+                }
+            }
+            return;
+        }
     }
     // flush: column i of rows M::row(k, 0 .. 3), within the tile
     if (i >= wv) return;
-    const long long plane = (long long)g.nu * g.nv;
     int gcol = tv * g.Tv + i + g.nv / 2;
     if (gcol >= g.nv) gcol -= g.nv;
 #pragma unroll
@@ -1644,37 +1758,40 @@ __device__ __forceinline__ void grid_item_mfma(Geo g, const Rec<T>* __restrict__
 
 // Waves per SIMD: four in single precision with one output (106 registers);
 // two where the accumulators take 128, one where they take 256.
-template <int S, bool FORM>
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4, 8))) void k_grid_mfma(Geo g, const Rec<float>* __restrict__ recs,
+constexpr int kMfmaWaves = 8;  // most waves an item in single precision
+extern __shared__ __align__(16) unsigned char mfma_smem[];
+
+template <int S, int NOUT, bool FORM>
+__global__ __launch_bounds__(64 * kMfmaWaves) __attribute__((amdgpu_waves_per_eu(NOUT == 2 ? 2 : 4, 8))) void k_grid_mfma(Geo g, const Rec<float>* __restrict__ recs,
                                                   const std::uint32_t* __restrict__ off,
                                                   const float* __restrict__ coeff, DevIn in, int G,
                                                   int ngroups, std::uint32_t rc,
                                                   const std::uint32_t* __restrict__ item_off,
                                                   const std::uint32_t* __restrict__ order,
                                                   cx<float>* __restrict__ grid) {
-    __shared__ MfmaShared<float, S, 1> sh;
-    grid_item_mfma<float, S, 1, FORM>(g, recs, off, coeff, in, G, ngroups, rc, item_off, order, grid, blockIdx.x,
-                                      sh.coef, sh.start, sh.pre, sh.rec, sh.unit, sh.qr);
+    __shared__ float coef[2 * ne_of<S>() * S];
+    grid_item_mfma<float, S, NOUT, FORM>(g, recs, off, coeff, in, G, ngroups, rc, item_off, order, grid, blockIdx.x,
+                                         coef, mfma_smem);
 }
 
-template <class T, int S, int NOUT, bool FORM>
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 8 && NOUT == 2 ? 1 : 2, 4))) void k_grid_mfma_wide(Geo g, const Rec<T>* __restrict__ recs,
+template <int S, int NOUT, bool FORM>
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(NOUT == 2 ? 1 : 2, 4))) void k_grid_mfma64(Geo g, const Rec<double>* __restrict__ recs,
                                                   const std::uint32_t* __restrict__ off,
-                                                  const T* __restrict__ coeff, DevIn in, int G,
+                                                  const double* __restrict__ coeff, DevIn in, int G,
                                                   int ngroups, std::uint32_t rc,
                                                   const std::uint32_t* __restrict__ item_off,
                                                   const std::uint32_t* __restrict__ order,
-                                                  cx<T>* __restrict__ grid) {
-    __shared__ MfmaShared<T, S, NOUT> sh;
-    grid_item_mfma<T, S, NOUT, FORM>(g, recs, off, coeff, in, G, ngroups, rc, item_off, order, grid, blockIdx.x,
-                                     sh.coef, sh.start, sh.pre, sh.rec, sh.unit, sh.qr);
+                                                  cx<double>* __restrict__ grid) {
+    __shared__ double coef[2 * ne_of<S>() * S];
+    grid_item_mfma<double, S, NOUT, FORM>(g, recs, off, coeff, in, G, ngroups, rc, item_off, order, grid, blockIdx.x,
+                                          coef, mfma_smem);
 }
 
 // Every job's items in one launch on the matrix cores (jobs as k_grid_jobs,
 // each gridded by the item body above at its support).
 template <bool FORM>
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4, 8))) void k_grid_mfma_jobs(const GridJob<float>* __restrict__ jobs, int njobs) {
-    __shared__ MfmaShared<float, 8, 1> sh;
+__global__ __launch_bounds__(64 * kMfmaWaves) __attribute__((amdgpu_waves_per_eu(4, 8))) void k_grid_mfma_jobs(const GridJob<float>* __restrict__ jobs, int njobs) {
+    __shared__ float coef[2 * ne_of<8>() * 8];
     int j = 0;
     for (int k = 1; k < njobs; ++k)
         if (jobs[k].first <= blockIdx.x) j = k;
@@ -1684,9 +1801,10 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4, 8))) void
 #define MJOB_CASE(SS)                                                                                    \
     case SS:                                                                                             \
         grid_item_mfma<float, SS, 1, FORM>(J.g, J.recs, J.off, J.coeff, J.in, J.G, J.ngroups, J.rc, J.item_off, \
-                                 J.order, J.grid, item, sh.coef, sh.start, sh.pre, sh.rec, sh.unit, sh.qr); \
+                                           J.order, J.grid, item, coef, mfma_smem); \
         break;
         MJOB_CASE(4) MJOB_CASE(5) MJOB_CASE(6) MJOB_CASE(7) MJOB_CASE(8)
+#undef MJOB_CASE
     default:
         break;
     }
@@ -1696,16 +1814,14 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4, 8))) void
 // registers to share one): the jobs of support S.
 template <int S>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 4))) void k_grid_mfma_jobs64(const GridJob<double>* __restrict__ jobs, int njobs) {
-    __shared__ MfmaShared<double, S, 1> sh;
+    __shared__ double coef[2 * ne_of<S>() * S];
     int j = 0;
     for (int k = 1; k < njobs; ++k)
         if (jobs[k].first <= blockIdx.x) j = k;
     const GridJob<double>& J = jobs[j];
     grid_item_mfma<double, S, 1, false>(J.g, J.recs, J.off, J.coeff, J.in, J.G, J.ngroups, J.rc, J.item_off, J.order,
-                                        J.grid, blockIdx.x - J.first, sh.coef, sh.start, sh.pre, sh.rec, sh.unit,
-                                        sh.qr);
+                                        J.grid, blockIdx.x - J.first, coef, mfma_smem);
 }
-#undef MJOB_CASE
 
 // ------------------------------------------------------------ transforms
 
@@ -2960,31 +3076,34 @@ void launch_grid(int S, int nblocks, std::size_t lds, hipStream_t st, const Geo&
 }
 
 template <class T>
-void launch_grid_mfma(int S, int nblocks, int nout, bool form, hipStream_t st, const Geo& g, const Rec<T>* recs,
-                      const std::uint32_t* off, const T* coeff, const DevIn& in, int G, int ngroups,
+void launch_grid_mfma(int S, int nblocks, int waves, int nout, bool form, hipStream_t st, const Geo& g,
+                      const Rec<T>* recs, const std::uint32_t* off, const T* coeff, const DevIn& in, int G, int ngroups,
                       std::uint32_t rc, const std::uint32_t* item_off, const std::uint32_t* order,
                       cx<T>* out) {
-#define MFMA_LAUNCH(KERNEL) \
-    KERNEL<<<nblocks, 64, 0, st>>>(g, recs, off, coeff, in, G, ngroups, rc, item_off, order, out)
-#define MFMA_CASE(SS)                                                                      \
-    case SS:                                                                               \
-        if constexpr (SS <= max_support<T>()) {                                            \
-            if (nout == 2) {                                                               \
-                MFMA_LAUNCH((k_grid_mfma_wide<T, SS, 2, false>));                          \
-            } else if constexpr (sizeof(T) == 4) {                                         \
-                if (form)                                                                  \
-                    MFMA_LAUNCH((k_grid_mfma<SS, true>));                                  \
-                else                                                                       \
-                    MFMA_LAUNCH((k_grid_mfma<SS, false>));                                 \
-            } else {                                                                       \
-                if (form)                                                                  \
-                    MFMA_LAUNCH((k_grid_mfma_wide<T, SS, 1, true>));                       \
-                else                                                                       \
-                    MFMA_LAUNCH((k_grid_mfma_wide<T, SS, 1, false>));                      \
-            }                                                                              \
-        } else {                                                                           \
-            throw DevError{"kernel support too large for this precision"};                 \
-        }                                                                                  \
+    const std::size_t lds = nout == 2 ? mfma_lds<T, 2>(g, G, waves) : mfma_lds<T, 1>(g, G, waves);
+#define MFMA_LAUNCH(SS, NO, FORM)                                                                                 \
+    do {                                                                                                          \
+        const auto kernel = [] {                                                                                  \
+            if constexpr (sizeof(T) == 4)                                                                         \
+                return k_grid_mfma<SS, NO, FORM>;                                                                 \
+            else                                                                                                  \
+                return k_grid_mfma64<SS, NO, FORM>;                                                               \
+        }();                                                                                                      \
+        lds_limit((const void*)kernel, lds);                                                                      \
+        kernel<<<nblocks, 64 * waves, lds, st>>>(g, recs, off, coeff, in, G, ngroups, rc, item_off, order, out);  \
+    } while (0)
+#define MFMA_CASE(SS)                                                      \
+    case SS:                                                               \
+        if constexpr (SS <= max_support<T>()) {                            \
+            if (nout == 2)                                                 \
+                MFMA_LAUNCH(SS, 2, false);                                 \
+            else if (form)                                                 \
+                MFMA_LAUNCH(SS, 1, true);                                  \
+            else                                                           \
+                MFMA_LAUNCH(SS, 1, false);                                 \
+        } else {                                                           \
+            throw DevError{"kernel support too large for this precision"}; \
+        }                                                                  \
         break;
     switch (S) {
         MFMA_CASE(4) MFMA_CASE(5) MFMA_CASE(6) MFMA_CASE(7) MFMA_CASE(8) MFMA_CASE(9) MFMA_CASE(10) MFMA_CASE(11)
@@ -2998,9 +3117,9 @@ void launch_grid_mfma(int S, int nblocks, int nout, bool form, hipStream_t st, c
 }
 
 void launch_jobs64(int S, int nblocks, hipStream_t st, const GridJob<double>* jobs, int njobs) {
-#define JOB64_CASE(SS)                                              \
-    case SS:                                                        \
-        k_grid_mfma_jobs64<SS><<<nblocks, 64, 0, st>>>(jobs, njobs); \
+#define JOB64_CASE(SS)                                                                                  \
+    case SS:                                                                                            \
+        k_grid_mfma_jobs64<SS><<<nblocks, 64, sizeof(MfmaWave<double, 1>), st>>>(jobs, njobs);          \
         break;
     switch (S) {
         JOB64_CASE(4) JOB64_CASE(5) JOB64_CASE(6) JOB64_CASE(7) JOB64_CASE(8) JOB64_CASE(9) JOB64_CASE(10)
@@ -3295,12 +3414,15 @@ int device_cus() {
     return std::max(n, 1);
 }
 
-// One count from the device (the stream is synchronised).
-long long read_u32(Workspace& ws, const std::uint32_t* d, hipStream_t st) {
-    std::uint32_t* h = static_cast<std::uint32_t*>(ws.host(sizeof(std::uint32_t)));
+// One count from the device (the stream is synchronised), or a second one too.
+long long read_u32(Workspace& ws, const std::uint32_t* d, hipStream_t st, const std::uint32_t* d2 = nullptr,
+                   long long* second = nullptr) {
+    std::uint32_t* h = static_cast<std::uint32_t*>(ws.host(2 * sizeof(std::uint32_t)));
     HIPCHK(hipMemcpyAsync(h, d, sizeof(std::uint32_t), hipMemcpyDeviceToHost, st));
+    if (d2) HIPCHK(hipMemcpyAsync(h + 1, d2, sizeof(std::uint32_t), hipMemcpyDeviceToHost, st));
     HIPCHK(hipStreamSynchronize(st));
-    return (long long)*h;
+    if (d2) *second = (long long)h[1];
+    return (long long)h[0];
 }
 
 template <class T, bool USE_VIS>
@@ -3342,17 +3464,31 @@ constexpr std::size_t grid_lds() {
 // once a split tile's chunks add only the cells they reach (gridding stage:
 // 512 -> 280.5 ms, 1024 -> 251.6, 2048 -> 238.0, 4096 -> 233.4, 8192 -> 234.5).
 constexpr std::uint32_t kGridChunk = 4096;
-// On the matrix cores an item is one wave's serial work, so a call of few
-// visibilities takes shorter ones: about kGridItems items over the whole call
-// (a visibility reaches two to four tiles' items), at least 128 records each.
-// Measured, items of 4096 records -> this rule: 118 k visibilities 545 -> 365
-// us (single precision, host arrays) and 1594 -> 1350 us (normal operator,
-// double precision), 3.2 M 1448 -> 1255 us; twice or half as many items are
-// within 3 % of it, four times as many slower (3.2 M: 1520 us).
+// On the matrix cores a wave takes records serially, so a call of few visibilities
+// spreads a tile's over more waves: about kGridItems over the whole call (a
+// visibility reaches two to four tiles' items), at least 128 records each.
+// Double precision takes shorter items for it. Single precision keeps its items
+// and gives each several waves, whose sums meet in LDS: every item of a split
+// tile adds into the grid in single precision, and 128 records an item made
+// that rounding four times what it is with 4096 (118 k visibilities on a few
+// tiles: 5.3e-7 -> 2.4e-6).
 constexpr long long kGridItems = 16384;
+std::uint32_t records_per_wave(long long n) {
+    return std::uint32_t(std::max<long long>(128, std::min<long long>(kGridChunk, 4 * n / kGridItems)));
+}
+template <class T>
 std::uint32_t grid_chunk(const Geo& g) {
-    if (!g.mfma) return kGridChunk;
-    return std::uint32_t(std::max<long long>(128, std::min<long long>(kGridChunk, 4 * g.n / kGridItems)));
+    return g.mfma && sizeof(T) == 8 ? records_per_wave(g.n) : kGridChunk;
+}
+// Waves an item over n visibilities. Two or three would leave half of a CU empty
+// beside the LDS of their sums; sums in double are always shared. Eight where
+// records are few, four otherwise (118 k visibilities: eight 381 us, four 403,
+// two 450; 3.2 M: 1291, 1205 and 1385).
+template <class T>
+int grid_waves(long long n, bool doubles) {
+    if (sizeof(T) == 8) return 1;
+    const std::uint32_t per = records_per_wave(n);
+    return per <= 256 ? 8 : per <= kGridChunk / 3 || doubles ? 4 : 1;
 }
 constexpr std::uint32_t kDegridChunk = 1024;     // visibilities per degridding item
 // Staged degridding holds a tile and its halo on every plane in LDS: in
@@ -3523,14 +3659,16 @@ bool fill_geo(const Geometry& G, Geo& g, int nout, bool degrid, std::string& err
     // precision with one output on multiples of 16 only: other tilings hold
     // more buckets, and calls near the block's limit would no longer fit.
     const int mu = mfma_tile(g.nu, g.supp), mv = mfma_tile(g.nv, g.supp);
-    const bool fits = fixed ? sizeof(T) == 4 && nout == 1 && g.nu % kMfmaTile == 0 && g.nv % kMfmaTile == 0
-                            : mu > 0 && mv > 0;
+    const bool single_sums = sizeof(T) == 4 && nout == 1 && g.nu % kMfmaTile == 0 && g.nv % kMfmaTile == 0;
+    const bool fits = fixed ? single_sums : mu > 0 && mv > 0;
     // degridding goes there in double precision where a tile's planes do not
     // fit the staged LDS form (3.2 M visibilities at 1024^2, support 11: 11.6
     // -> 4.8 ms; support 7, which fits, 1.7 ms staged and 3.0 ms there); in
     // single precision the staged form is the faster one throughout
     const bool unstaged = sizeof(T) == 8 && degrid_lds<T>(g.Tu, g.Tv, g.supp, P) > degrid_lds_max<T>();
-    g.mfma = (!degrid || unstaged) && g.wgrid && g.supp <= max_support<T>() && tile == 0 && fits && mfma_enabled() ? 1 : 0;
+    g.mfma = (!degrid || unstaged) && g.wgrid && g.supp <= max_support<T>() && tile == 0 && fits && mfma_enabled()
+                 ? (single_sums ? kMfmaSingle : kMfmaDouble)
+                 : 0;
     if (g.mfma) {
         g.Tu = mu;
         g.Tv = mv;
@@ -4065,6 +4203,7 @@ struct GridPrep {
     LongTabs<T> lt;
     int P = 0, G_planes = 0, ngroups = 0, ntg = 0, TvP = 0;
     std::uint32_t rc = kGridChunk;  // visibilities per item
+    int waves = 1;                  // per workgroup on the matrix cores
     std::size_t lds = 0;
     std::uint32_t* item_off = nullptr;
     long long ub = 0;  // workgroups of the gridding launch
@@ -4073,10 +4212,11 @@ struct GridPrep {
 };
 
 // Tables, the grid (its cells reached by several items cleared) and the
-// work items of one vis2dirty of `nout` outputs.
+// work items of one vis2dirty of `nout` outputs, for workgroups of `waves` on
+// the matrix cores.
 template <class T>
 void grid_prepare(Workspace& ws, const Geometry& G, const Geo& g, const std::uint32_t* off, int nout,
-                  hipStream_t st, HostKeep& keep, StageTimer& timer, ItemCache* cache, GridPrep<T>& gp) {
+                  hipStream_t st, HostKeep& keep, StageTimer& timer, ItemCache* cache, GridPrep<T>& gp, int waves) {
     make_tables<T>(ws, G, g, st, keep, gp.tb, 0);
     make_long<T>(ws, g, st, keep, gp.lt);
     timer.mark("tables");
@@ -4098,43 +4238,52 @@ void grid_prepare(Workspace& ws, const Geometry& G, const Geo& g, const std::uin
         gp.G_planes = std::max(1, std::min({P, int(grid_lds<T>() / per_plane), 32}));
         gp.lds = per_plane * std::min(P, gp.G_planes);
     }
-    gp.rc = grid_chunk(g);
+    gp.rc = grid_chunk<T>(g);
     gp.ngroups = (P + gp.G_planes - 1) / gp.G_planes;
     gp.ntg = g.ntu * g.ntv * gp.ngroups;
     const int ntg = gp.ntg;
-    std::uint32_t* items = static_cast<std::uint32_t*>(ws.get(kSlotItems, sizeof(std::uint32_t) * (ntg + 1)));
-    gp.item_off = static_cast<std::uint32_t*>(ws.get(kSlotItemOff, sizeof(std::uint32_t) * (ntg + 1)));
+    gp.waves = g.mfma ? waves : 1;
+    const int split = gp.waves > 1 ? 1 : 0;
+    const std::size_t nunits = std::size_t(ntg) * (split ? 2 : 1);
+    std::uint32_t* items = static_cast<std::uint32_t*>(ws.get(kSlotItems, sizeof(std::uint32_t) * (nunits + 1)));
+    gp.item_off = static_cast<std::uint32_t*>(ws.get(kSlotItemOff, sizeof(std::uint32_t) * (nunits + 1)));
     if (!cache || !cache->valid) {
         k_grid_items<<<(ntg + 1 + 255) / 256, 256, 0, st>>>(g, off, gp.tb.order, gp.G_planes, gp.ngroups, g.supp,
-                                                             gp.rc, items);
+                                                             gp.rc, split, items);
         HIPCHK(hipGetLastError());
-        exclusive_scan(ws, items, gp.item_off, ntg + 1, st);
+        exclusive_scan(ws, items, gp.item_off, (long long)nunits + 1, st);
     }
     // the in-LDS row transform reads only the tiles an item reached
     // (RANG_GRID_OCC=0: every cell cleared and read)
     gp.occ = nullptr;
     if (!g.lv1 && grid_occ(sizeof(cx<T>) * std::size_t(plane) * P)) {
         std::uint8_t* occ = static_cast<std::uint8_t*>(ws.get(kSlotOcc, std::size_t(ntg)));
-        k_occupancy<<<(ntg + 255) / 256, 256, 0, st>>>(gp.item_off, gp.tb.order, ntg, gp.ngroups, g.ntu * g.ntv, occ);
+        k_occupancy<<<(ntg + 255) / 256, 256, 0, st>>>(gp.item_off, gp.tb.order, ntg, gp.ngroups, g.ntu * g.ntv, split,
+                                                           occ);
         HIPCHK(hipGetLastError());
         gp.occ = occ;
     }
     const int skip = gp.occ ? 1 : 0;
     if (nout == 2)
-        k_zero_split<T, 2><<<ntg, 256, 0, st>>>(g, gp.item_off, gp.tb.order, gp.G_planes, gp.ngroups, gp.grid, skip);
+        k_zero_split<T, 2><<<ntg, 256, 0, st>>>(g, gp.item_off, gp.tb.order, gp.G_planes, gp.ngroups, gp.grid, skip,
+                                               split);
     else
-        k_zero_split<T, 1><<<ntg, 256, 0, st>>>(g, gp.item_off, gp.tb.order, gp.G_planes, gp.ngroups, gp.grid, skip);
+        k_zero_split<T, 1><<<ntg, 256, 0, st>>>(g, gp.item_off, gp.tb.order, gp.G_planes, gp.ngroups, gp.grid, skip,
+                                               split);
     HIPCHK(hipGetLastError());
     if (cache && cache->valid) {
         gp.ub = cache->ub;
     } else {
-        gp.ub = read_u32(ws, gp.item_off + ntg, st);
+        // a workgroup per long item, then one per `waves` short ones
+        long long all = 0;
+        gp.ub = read_u32(ws, gp.item_off + ntg, st, split ? gp.item_off + nunits : nullptr, &all);
+        if (split) gp.ub += (all - gp.ub + gp.waves - 1) / gp.waves;
         if (cache) {
             cache->ub = gp.ub;
             cache->valid = true;
         }
     }
-    if (gp.ub >= (1LL << 31)) throw DevError{"too many gridding items"};
+    if (gp.ub >= (1LL << 31) || gp.ub * 64 * gp.waves >= (1LL << 32)) throw DevError{"too many gridding items"};
 }
 
 // The transforms of the gridded planes and their corrected sum into `dirty`
@@ -4213,12 +4362,12 @@ void grid_pipeline(Workspace& ws, const Geometry& G, const Geo& g, const DevIn& 
                    const Rec<T>* recs, const std::uint32_t* off, int nout, bool form, T* dirty,
                    T* psf, hipStream_t st, HostKeep& keep, StageTimer& timer, ItemCache* cache = nullptr) {
     GridPrep<T> gp;
-    grid_prepare<T>(ws, G, g, off, nout, st, keep, timer, cache, gp);
+    grid_prepare<T>(ws, G, g, off, nout, st, keep, timer, cache, gp, grid_waves<T>(g.n, g.mfma == kMfmaDouble));
     const std::uint32_t rc = gp.rc;
     if (gp.ub == 0) {
         // nothing to grid: every cell was cleared above
     } else if (g.mfma) {
-        launch_grid_mfma<T>(g.supp, int(gp.ub), nout, form, st, g, recs, off, gp.tb.coeff, din, gp.G_planes,
+        launch_grid_mfma<T>(g.supp, int(gp.ub), gp.waves, nout, form, st, g, recs, off, gp.tb.coeff, din, gp.G_planes,
                             gp.ngroups, rc, gp.item_off, gp.tb.order, gp.grid);
     } else if (nout == 2)
         launch_grid<T, 2, false>(g.supp, int(gp.ub), gp.lds, st, g, recs, off, gp.tb.coeff, din, gp.G_planes,
@@ -4593,6 +4742,17 @@ int device_batch_vis2dirty(BatchImage* imgs, int n, std::size_t budget, hipStrea
             std::size_t lds = 0;
             long long total = 0;
             std::map<int, long long> mtotal;
+            // the images on the matrix cores share a launch
+            long long mvis = 0;
+            bool mdouble = false;
+            int mg = 0;
+            for (std::size_t k = at; k < end; ++k) {
+                const Geo& g = plans[order[k]].g;
+                if (!g.mfma) continue;
+                mvis += g.n;
+                mdouble |= g.mfma == kMfmaDouble;
+            }
+            const int waves = grid_waves<T>(mvis, mdouble);
             for (std::size_t k = at; k < end; ++k) {
                 const int i = order[k];
                 Plan& pl = plans[i];
@@ -4602,16 +4762,19 @@ int device_batch_vis2dirty(BatchImage* imgs, int n, std::size_t budget, hipStrea
                 std::uint32_t* off;
                 sort_records<T, 0, true>(ws, pl.din, pl.g, pl.nvis, st, &recs, &off);
                 GridPrep<T>& gp = preps[k - at];
-                grid_prepare<T>(ws, pl.G, pl.g, off, 1, st, keep, timer, nullptr, gp);
+                grid_prepare<T>(ws, pl.G, pl.g, off, 1, st, keep, timer, nullptr, gp, waves);
                 if (gp.ub == 0) continue;
                 const int kind = sizeof(T) == 4 ? 0 : pl.g.supp;
                 long long& tot = pl.g.mfma ? mtotal[kind] : total;
-                if (tot + gp.ub >= (1LL << 31)) throw DevError{"too many gridding items in one batch"};
+                if (tot + gp.ub >= (1LL << 31) || (tot + gp.ub) * 64 * gp.waves >= (1LL << 32)) throw DevError{"too many gridding items in one batch"};
                 (pl.g.mfma ? mjobs[kind] : jobs)
                     .push_back(GridJob<T>{pl.g, recs, off, gp.tb.coeff, pl.din, gp.G_planes, gp.ngroups, gp.TvP,
                                           gp.rc, gp.item_off, gp.tb.order, gp.grid, std::uint32_t(tot)});
                 tot += gp.ub;
-                if (!pl.g.mfma) lds = std::max(lds, gp.lds);
+                if (!pl.g.mfma)
+                    lds = std::max(lds, gp.lds);
+                else
+                    mg = std::max(mg, gp.G_planes);
             }
             timer.mark("sort");
             // the job tables to the device: one launch per gridding kernel
@@ -4636,7 +4799,9 @@ int device_batch_vis2dirty(BatchImage* imgs, int n, std::size_t budget, hipStrea
                 const GridJob<T>* d = upload(m.second);
                 const int njobs = int(m.second.size()), blocks = int(mtotal[m.first]);
                 if constexpr (sizeof(T) == 4) {
-                    k_grid_mfma_jobs<false><<<blocks, 64, 0, st>>>(d, njobs);
+                    const std::size_t mlds = mfma_lds<T, 1>(m.second[0].g, mg, waves);
+                    lds_limit((const void*)k_grid_mfma_jobs<false>, mlds);
+                    k_grid_mfma_jobs<false><<<blocks, 64 * waves, mlds, st>>>(d, njobs);
                     HIPCHK(hipGetLastError());
                 } else {
                     launch_jobs64(m.first, blocks, st, d, njobs);
