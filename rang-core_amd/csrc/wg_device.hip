@@ -2359,10 +2359,17 @@ __global__ __launch_bounds__(NT) void k_cols_fwd(const T* __restrict__ img,
     }
 }
 
+// Waves per SIMD that k_rows_fwd is built for, at least: lines of 1025 to 2048
+// doubles would take 225 registers, two waves, where four fit beside their LDS.
+template <class T, int NT, int MAXTOT>
+constexpr int rows_fwd_waves() {
+    return sizeof(T) == 8 && MAXTOT == 2048 ? 4 : NT / 256;
+}
+
 // d2v: one grid row from its image columns, forward transform along v
 // (wgridder.rs:2922-2929, 2968-2991).
 template <class T, int NT, int MAXTOT>
-__global__ __launch_bounds__(NT) void k_rows_fwd(const cx<T>* __restrict__ tmp,
+__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(rows_fwd_waves<T, NT, MAXTOT>()))) void k_rows_fwd(const cx<T>* __restrict__ tmp,
                                                           cx<T>* __restrict__ grid, FftDesc d,
                                                           const cx<T>* __restrict__ tw, Geo g,
                                                           const std::uint8_t* __restrict__ need) {
