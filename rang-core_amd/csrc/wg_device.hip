@@ -3659,15 +3659,20 @@ bool fill_geo(const Geometry& G, Geo& g, int nout, bool degrid, std::string& err
         err = "no tile size divides the grid";
         return false;
     }
-    // w-gridding goes to the matrix cores where the axes tile for them,
-    // unless a tile side is asked for (measured against the LDS gridder:
-    // 3.2 M visibilities, support 6, single precision 1227 -> 517 us; double
-    // precision at k_grid_mfma_wide). In the fixed scratch block, single
-    // precision with one output on multiples of 16 only: other tilings hold
-    // more buckets, and calls near the block's limit would no longer fit.
+    // w-gridding goes to the matrix cores where the axes tile for them, unless a
+    // tile side is asked for (figures at grid_item_mfma). With double sums from
+    // support 5 on: at 4 a 16-cell window takes 256 products for 16 useful ones, and
+    // the LDS gridder is the faster one for dense data (one output of 19.4 M
+    // visibilities in double precision 3.8 ms there, 4.8 here; two in single 3.9 and
+    // 4.8; support 5: 7.0 and 5.8, 10.2 and 5.8). Two single-precision outputs of
+    // support 5 from 2^20 visibilities on: thinly spread, 118 k to 806 k take 0.91 to
+    // 0.93 of the time in LDS, 1.6 M 1.12. In the fixed scratch block, single
+    // precision with one output on multiples of 16 only: other tilings hold more
+    // buckets, and calls near the block's limit would no longer fit.
     const int mu = mfma_tile(g.nu, g.supp), mv = mfma_tile(g.nv, g.supp);
     const bool single_sums = sizeof(T) == 4 && nout == 1 && g.nu % kMfmaTile == 0 && g.nv % kMfmaTile == 0;
-    const bool fits = fixed ? single_sums : mu > 0 && mv > 0;
+    const bool wide = g.supp >= 6 || (g.supp == 5 && (sizeof(T) == 8 || nout == 1 || g.n >= (1LL << 20)));
+    const bool fits = fixed ? single_sums : mu > 0 && mv > 0 && (degrid || single_sums || wide);
     // degridding goes there in double precision where a tile's planes do not
     // fit the staged LDS form (3.2 M visibilities at 1024^2, support 11: 11.6
     // -> 4.8 ms; support 7, which fits, 1.7 ms staged and 3.0 ms there); in
