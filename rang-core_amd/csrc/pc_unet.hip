@@ -11,17 +11,20 @@
 // and the master weights are FP32.
 //
 // A 3 x 3 convolution is an implicit GEMM on v_mfma_f32_16x16x32_bf16 with the
-// image tile and its halo in LDS (k_conv3_fwd, k_conv3_wgrad below); the 1 x 1
-// output convolution, which only streams its tensors, keeps a per-wave kernel
-// on v_mfma_f32_16x16x16_bf16 (16 pixels x 32 output channels, operands read
-// from memory). Channel counts are multiples of 16 (callers pad the first and
+// image tile and its halo in LDS (k_conv3_fwd, k_conv_wgrad below); the 1 x 1
+// output convolution, which only streams its tensors, and layers too small for
+// the tiles take per-wave kernels on v_mfma_f32_16x16x16_bf16 (16 pixels x 32
+// output channels, operands read from memory). Channel counts are multiples of 16 (callers pad the first and
 // last layers).
 
 #include <hip/hip_runtime.h>
 
 #include <cmath>
 #include <cstdint>
+#include <map>
+#include <mutex>
 #include <string>
+#include <utility>
 
 #include "../../include/rang_core_precond.h"
 
@@ -62,31 +65,49 @@ __device__ __forceinline__ bf16x4 load4(const std::uint16_t* p, bool ok) {
     return r;
 }
 
-// y = conv1x1(x, w) over npix pixels: w as [cout][cin] BF16; the FP32 result
-// into y (pre-activation, may be null) and BF16 relu(y) (or y when relu is 0)
-// into a (may be null). Block: 4 waves, 64 pixels x 32 output channels. A row
-// = pixel (lane mod 16), k = 4 consecutive input channels per lane group
-// (lane / 16); B column = output channel, the same k split; D column = output
-// channel (lane mod 16), rows 4 (lane / 16) + t.
-__global__ __launch_bounds__(256) void k_conv1_fwd(const std::uint16_t* __restrict__ x, int ldx, int xoff,
-                                                   const std::uint16_t* __restrict__ w, float* __restrict__ y,
-                                                   std::uint16_t* __restrict__ a, int ldy, int yoff, long long npix,
-                                                   int cin, int cout, int relu) {
+// y = conv(x, w) over B images of H x W: w as [cout][ks * ks][cin] BF16; the
+// FP32 result into y (pre-activation, may be null) and BF16 relu(y) (or y
+// when relu is 0) into a (may be null). Block: 4 waves, 64 pixels x 32 output
+// channels, every operand read from memory: for 1 x 1 and for small 3 x 3
+// convolutions (small_fwd). A row = pixel (lane mod 16), k = 4 consecutive input
+// channels per lane group (lane / 16); B column = output channel, the same k
+// split; D column = output channel (lane mod 16), rows 4 (lane / 16) + t.
+template <int KS>
+__global__ __launch_bounds__(256) void k_conv_fwd_wave(const std::uint16_t* __restrict__ x, int ldx, int xoff,
+                                                       const std::uint16_t* __restrict__ w, float* __restrict__ y,
+                                                       std::uint16_t* __restrict__ a, int ldy, int yoff, int B,
+                                                       int H, int W, int cin, int cout, int relu) {
+    const long long npix = (long long)B * H * W;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const long long p0 = (long long)blockIdx.x * 64 + wave * 16;
     const int co0 = blockIdx.y * 32;
     const int row = lane & 15, q = lane >> 4;
-    const bool in = p0 + row < npix;
-    const std::uint16_t* xa = x + (p0 + row) * ldx + xoff + 4 * q;
-    const std::uint16_t* wb0 = w + (long long)(co0 + row) * cin + 4 * q;
-    const std::uint16_t* wb1 = wb0 + 16LL * cin;
+    // this lane's A pixel
+    const long long pa = p0 + row;
+    int n = 0, h = 0, wc = 0;
+    if (pa < npix) {
+        n = int(pa / ((long long)H * W));
+        const int r = int(pa - (long long)n * H * W);
+        h = r / W;
+        wc = r - h * W;
+    }
     f32x4 acc0 = {0.f, 0.f, 0.f, 0.f}, acc1 = {0.f, 0.f, 0.f, 0.f};
-    for (int c0 = 0; c0 < cin; c0 += 16) {
-        const bf16x4 av = load4(xa + c0, in);
-        const bf16x4 b0 = load4(wb0 + c0, true);
-        const bf16x4 b1 = load4(wb1 + c0, co0 + 16 < cout);
-        acc0 = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(av, b0, acc0, 0, 0, 0);
-        acc1 = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(av, b1, acc1, 0, 0, 0);
+    constexpr int T = KS * KS;
+    for (int tap = 0; tap < T; ++tap) {
+        const int dy = KS == 3 ? tap / 3 - 1 : 0, dx = KS == 3 ? tap % 3 - 1 : 0;
+        const int hh = h + dy, ww = wc + dx;
+        const bool in = pa < npix && hh >= 0 && hh < H && ww >= 0 && ww < W;
+        const long long src = ((long long)n * H + hh) * W + ww;
+        const std::uint16_t* xa = x + src * ldx + xoff + 4 * q;
+        const std::uint16_t* wb0 = w + ((long long)(co0 + row) * T + tap) * cin + 4 * q;
+        const std::uint16_t* wb1 = w + ((long long)(co0 + 16 + row) * T + tap) * cin + 4 * q;
+        for (int c0 = 0; c0 < cin; c0 += 16) {
+            const bf16x4 av = load4(xa + c0, in);
+            const bf16x4 b0 = load4(wb0 + c0, true);
+            const bf16x4 b1 = load4(wb1 + c0, co0 + 16 < cout);
+            acc0 = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(av, b0, acc0, 0, 0, 0);
+            acc1 = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(av, b1, acc1, 0, 0, 0);
+        }
     }
 #pragma unroll
     for (int t = 0; t < 4; ++t) {
@@ -101,6 +122,54 @@ __global__ __launch_bounds__(256) void k_conv1_fwd(const std::uint16_t* __restri
             if (y) y[at] = v;
             if (a) a[at] = to_bf16(relu ? fmaxf(v, 0.f) : v);
         }
+    }
+}
+
+// dw += sum over pixels of dy (x) the shifted input, dw as [cout][ks * ks][cin]
+// FP32: a GEMM over pixels (16 per MFMA) for one (16 cout, tap, 16 cin)
+// tile per wave; each block sums a chunk of pixels and adds its tile. For few
+// pixels (small_wgrad).
+template <int KS>
+__global__ __launch_bounds__(256) void k_conv_wgrad_wave(const std::uint16_t* __restrict__ x, int ldx, int xoff,
+                                                         const std::uint16_t* __restrict__ dy, int lddy, int dyoff,
+                                                         float* __restrict__ dw, int B, int H, int W, int cin,
+                                                         int cout, long long chunk) {
+    constexpr int T = KS * KS;
+    const long long npix = (long long)B * H * W;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int nct = cin / 16, ncot = cout / 16;
+    const int tile = blockIdx.x * 4 + wave;  // (cout tile, tap, cin tile)
+    if (tile >= ncot * T * nct) return;
+    const int cot = tile / (T * nct), rem = tile - cot * T * nct;
+    const int tap = rem / nct, ct = rem - tap * nct;
+    const int ddy = KS == 3 ? tap / 3 - 1 : 0, ddx = KS == 3 ? tap % 3 - 1 : 0;
+    const int row = lane & 15, q = lane >> 4;
+    const long long pbeg = (long long)blockIdx.y * chunk, pend = pbeg + chunk < npix ? pbeg + chunk : npix;
+    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+    for (long long pb = pbeg; pb < pend; pb += 16) {
+        bf16x4 av, bv;
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+            const long long p = pb + 4 * q + t;
+            short va = 0, vb = 0;
+            if (p < pend) {
+                va = short(dy[p * lddy + dyoff + cot * 16 + row]);
+                const int n = int(p / ((long long)H * W));
+                const int r = int(p - (long long)n * H * W);
+                const int hh = r / W + ddy, ww = r % W + ddx;
+                if (hh >= 0 && hh < H && ww >= 0 && ww < W)
+                    vb = short(x[(((long long)n * H + hh) * W + ww) * ldx + xoff + ct * 16 + row]);
+            }
+            av[t] = va;
+            bv[t] = vb;
+        }
+        acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(av, bv, acc, 0, 0, 0);
+    }
+    // D row = cout within the tile (4 q + t), column = cin within the tile (row)
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+        const int co = cot * 16 + 4 * q + t, ci = ct * 16 + row;
+        atomicAdd(&dw[((long long)co * T + tap) * cin + ci], acc[t]);
     }
 }
 
@@ -836,18 +905,59 @@ bool vector8(const E* p, int ld, int off) {
     return reinterpret_cast<std::uintptr_t>(p) % 16 == 0 && ld % unit == 0 && off % unit == 0;
 }
 
+// Lets `kernel` take `bytes` of dynamic LDS on this device, once.
+int lds_once(const void* kernel, std::size_t bytes) {
+    static std::mutex mu;
+    static std::map<std::pair<int, const void*>, std::size_t> done;
+    int dev = 0;
+    if (const int e = nn_fail(hipGetDevice(&dev))) return e;
+    std::lock_guard<std::mutex> lk(mu);
+    std::size_t& had = done[{dev, kernel}];
+    if (had >= bytes) return 0;
+    if (const int e = nn_fail(hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, int(bytes))))
+        return e;
+    had = bytes;
+    return 0;
+}
+
+// Workgroups of the tiled forward product, without the output channels.
+template <int WCO>
+long long conv3_tiles(int B, int H, int W) {
+    const int rows = Conv3Tile<WCO>::rows;
+    return (long long)B * ((H + rows - 1) / rows) * ((W + kConvCols - 1) / kConvCols);
+}
+long long wgrad_tiles(int B, int H, int W) {
+    return (long long)B * ((H + kWgRows - 1) / kWgRows) * ((W + 31) / 32);
+}
+
+// Whether a layer goes to the per-wave kernels: few workgroups of tiles take
+// several times the few microseconds of a launch, the more so where the image
+// fills little of its tiles. Measured, per wave / in tiles, us. Forward: 32 -> 32
+// channels of 16384 pixels 6.4 / 11.3, 96 -> 32 12.6 / 22.5, 64 -> 64 (2^26
+// products a tap) equal; 512 images of 2 x 2, 256 -> 256, 40 / 171, of 4 x 4 172 /
+// 176. Weight gradient: 32 x 32 channels of 4096 pixels 10 / 18, 96 x 32 18.2 /
+// 18.4, 256 x 256 of 64 pixels 9.8 / 20.4, of 512 images of 2 x 2 125 / 279; 1 x 1:
+// 2048 pixels 4.7 / 5.4, 4096 9.0 / 5.2.
+bool small_fwd(int B, int H, int W, int cin, int cout) {
+    const double npix = double(B) * H * W;
+    const double tiled = cout % 64 == 0 ? 256.0 * conv3_tiles<2>(B, H, W) : 512.0 * conv3_tiles<1>(B, H, W);
+    return npix * cin * cout < 67108864.0 * (1.0 + tiled / npix / 16.0);
+}
+bool small_wgrad(int B, int H, int W, int cin, int cout, int ks) {
+    const double npix = double(B) * H * W;
+    if (ks == 1) return npix <= 2048.0;
+    return npix * cin * cout <= 4194304.0 * (2.0 + 256.0 * wgrad_tiles(B, H, W) / npix);
+}
+
 template <int WCO>
 int32_t conv3_launch(const std::uint16_t* x, int ldx, int xoff, const std::uint16_t* w, float* y, std::uint16_t* a, int ldy,
                             int yoff, int B, int H, int W, int cin, int cout, int relu, int unit, int out16,
                             hipStream_t st) {
     using Tile = Conv3Tile<WCO>;
     const int nth = (H + Tile::rows - 1) / Tile::rows, ntw = (W + kConvCols - 1) / kConvCols;
-    const long long blocks = (long long)B * nth * ntw;
-    if (blocks * 256 >= (1LL << 32)) return g_nn_err = "too many pixels for one convolution", 1;
+    const long long blocks = conv3_tiles<WCO>(B, H, W);
     const auto kernel = k_conv3_fwd<WCO>;
-    if (const int e = nn_fail(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
-                                                  hipFuncAttributeMaxDynamicSharedMemorySize, int(Tile::lds))))
-        return e;
+    if (const int e = lds_once(reinterpret_cast<const void*>(kernel), Tile::lds)) return e;
     kernel<<<dim3(unsigned(blocks), unsigned((cout + Tile::co - 1) / Tile::co)), 256, Tile::lds, st>>>(
         x, ldx, xoff, w, y, a, ldy, yoff, H, W, cin, cout, relu, nth, ntw, unit, out16);
     return nn_fail(hipGetLastError());
@@ -857,17 +967,14 @@ template <int KS, int WCO, int WCI>
 int32_t wgrad_launch(const std::uint16_t* x, int ldx, int xoff, const std::uint16_t* dy, int lddy, int dyoff, float* dw,
                             int B, int H, int W, int cin, int cout, hipStream_t st) {
     const int nth = (H + kWgRows - 1) / kWgRows, ntw = (W + 31) / 32;
-    const long long ntiles = (long long)B * nth * ntw;
-    if (ntiles >= (1LL << 30)) return g_nn_err = "too many pixels for one weight gradient", 1;
+    const long long ntiles = wgrad_tiles(B, H, W);
     const int nco = (cout + 32 * WCO - 1) / (32 * WCO), nci = (cin + 32 * WCI - 1) / (32 * WCI);
     // a workgroup per CU (its LDS), each with its share of the tiles
     const long long want = (256 + nco * nci - 1) / (nco * nci);
     const unsigned nwg = unsigned(ntiles < want ? ntiles : want);
     const std::size_t lds = WgradTile<KS>::lds(32 * WCI, 32 * WCO);
     const auto kernel = k_conv_wgrad<KS, WCO, WCI>;
-    if (const int e = nn_fail(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
-                                                  hipFuncAttributeMaxDynamicSharedMemorySize, int(lds))))
-        return e;
+    if (const int e = lds_once(reinterpret_cast<const void*>(kernel), lds)) return e;
     kernel<<<dim3(nwg, unsigned(nco * nci)), kWgThreads, lds, st>>>(x, ldx, xoff, dy, lddy, dyoff, dw, H, W, cin, cout, nth,
                                                             ntw, int(ntiles), nci, unit_of(x, ldx, xoff),
                                                             unit_of(dy, lddy, dyoff));
@@ -903,10 +1010,15 @@ int32_t rang_amd_nn_conv_fwd(const uint16_t* x, int32_t ldx, int32_t xoff, const
     if (const int e = conv_args_ok(ldx, xoff, ldy, yoff, cin, cout, ks)) return e;
     if (!x || !w || (!y && !a) || B <= 0 || H <= 0 || W <= 0) return g_nn_err = "null array or empty image", 1;
     hipStream_t st = static_cast<hipStream_t>(stream);
-    if (ks == 1) {
+    // thin images have more tiles than a launch can hold
+    const bool many = (cout % 64 == 0 ? conv3_tiles<2>(B, H, W) : conv3_tiles<1>(B, H, W)) >= (1LL << 24);
+    if (ks == 1 || many || small_fwd(B, H, W, cin, cout)) {
         const long long npix = (long long)B * H * W;
         const dim3 grid(unsigned((npix + 63) / 64), unsigned((cout + 31) / 32));
-        k_conv1_fwd<<<grid, 256, 0, st>>>(x, ldx, xoff, w, y, a, ldy, yoff, npix, cin, cout, relu);
+        if (ks == 3)
+            k_conv_fwd_wave<3><<<grid, 256, 0, st>>>(x, ldx, xoff, w, y, a, ldy, yoff, B, H, W, cin, cout, relu);
+        else
+            k_conv_fwd_wave<1><<<grid, 256, 0, st>>>(x, ldx, xoff, w, y, a, ldy, yoff, B, H, W, cin, cout, relu);
         return nn_fail(hipGetLastError());
     }
     const int ux = unit_of(x, ldx, xoff), uw = unit_of(w, 8, 0), unit = ux < uw ? ux : uw;
@@ -925,6 +1037,22 @@ int32_t rang_amd_nn_conv_wgrad(const uint16_t* x, int32_t ldx, int32_t xoff, con
     if (const int e = conv_args_ok(ldx, xoff, lddy, dyoff, cin, cout, ks)) return e;
     if (!x || !dy || !dw || B <= 0 || H <= 0 || W <= 0) return g_nn_err = "null array or empty image", 1;
     hipStream_t st = static_cast<hipStream_t>(stream);
+    if (wgrad_tiles(B, H, W) >= (1LL << 30) || small_wgrad(B, H, W, cin, cout, ks)) {
+        const long long npix = (long long)B * H * W;
+        const int tiles = (cout / 16) * ks * ks * (cin / 16);
+        // pixel chunks: enough blocks to fill the chip, chunks a multiple of 16
+        long long nchunk = (2048 + (tiles + 3) / 4 - 1) / ((tiles + 3) / 4);
+        if (nchunk < 1) nchunk = 1;
+        long long chunk = (npix + nchunk - 1) / nchunk;
+        chunk = (chunk + 15) / 16 * 16;
+        nchunk = (npix + chunk - 1) / chunk;
+        const dim3 grid(unsigned((tiles + 3) / 4), unsigned(nchunk));
+        if (ks == 3)
+            k_conv_wgrad_wave<3><<<grid, 256, 0, st>>>(x, ldx, xoff, dy, lddy, dyoff, dw, B, H, W, cin, cout, chunk);
+        else
+            k_conv_wgrad_wave<1><<<grid, 256, 0, st>>>(x, ldx, xoff, dy, lddy, dyoff, dw, B, H, W, cin, cout, chunk);
+        return nn_fail(hipGetLastError());
+    }
     const bool wo = cout % 64 == 0, wi = cin % 64 == 0;
     if (ks == 3) {
         if (wo && wi) return wgrad_launch<3, 2, 2>(x, ldx, xoff, dy, lddy, dyoff, dw, B, H, W, cin, cout, st);

@@ -130,6 +130,44 @@ def test_conv3_tile_edges(cin, cout, H, W, pad):
     assert float((torch_weight(dw.cpu(), 3).double() - ref_dw).abs().max()) <= bound
 
 
+# the tiled kernels' edges in layers large enough for them, and thin images, which
+# leave most of a tile empty and go to the per-wave kernels
+@pytest.mark.parametrize("cin,cout,B,H,W,pad", [
+    (16, 32, 1, 397, 401, 0), (48, 64, 3, 97, 95, 4), (96, 32, 2, 113, 127, 8), (64, 128, 1, 103, 99, 0),
+    (80, 48, 1, 137, 159, 4), (256, 256, 1, 33, 36, 0), (64, 64, 700, 5, 5, 0), (32, 32, 600, 2, 3, 0),
+])
+def test_conv3_large_layers(cin, cout, B, H, W, pad):
+    from rang import precond as P
+
+    lib, st = P._lib(), P._stream()
+    g = torch.Generator().manual_seed(cin + cout + B + H + W)
+    x, dy = torch.randn(B * H * W, cin + pad, generator=g), torch.randn(B * H * W, cout + pad, generator=g)
+    w = torch.randn(cout, 9, cin, generator=g) / math.sqrt(9 * cin)
+    xb, wb, dyb = bf16_bits(x).cuda(), bf16_bits(w).cuda(), bf16_bits(dy).cuda()
+    y = torch.full((B * H * W, cout + pad), 7.0, device="cuda")
+    a = torch.full((B * H * W, cout + pad), 5, dtype=torch.int16, device="cuda")
+    P._ok(lib.rang_amd_nn_conv_fwd(P._p(xb), cin + pad, pad, P._p(wb), P._p(y), P._p(a), cout + pad, pad, B, H, W, cin,
+                                   cout, 3, 1, st))
+    dw = torch.ones(cout, 9, cin, device="cuda")
+    P._ok(lib.rang_amd_nn_conv_wgrad(P._p(xb), cin + pad, pad, P._p(dyb), cout + pad, pad, P._p(dw), B, H, W, cin,
+                                     cout, 3, st))
+    xr = nchw(from_bits(xb.cpu())[:, pad:].contiguous(), B, H, W, cin).double()
+    dyr = nchw(from_bits(dyb.cpu())[:, pad:].contiguous(), B, H, W, cout).double()
+    wr = torch_weight(from_bits(wb.cpu()), 3).double()
+    got = nchw(y.cpu()[:, pad:].contiguous(), B, H, W, cout).double()
+    # FP32 sums of 9 cin (forward) and B H W (gradient) exact products: each
+    # addition rounds by 2^-24 of the sum of magnitudes
+    bound = 9 * cin * 2.0 ** -24 * float(F.conv2d(xr.abs(), wr.abs(), padding=1).max())
+    assert float((got - F.conv2d(xr, wr, padding=1)).abs().max()) <= bound
+    act = bf16_bits(y.cpu()[:, pad:].clamp(min=0))
+    assert torch.equal(a.cpu()[:, pad:], act)
+    assert bool((y.cpu()[:, :pad] == 7.0).all()) and bool((a.cpu()[:, :pad] == 5).all())
+    ref_dw = torch.nn.grad.conv2d_weight(xr, wr.shape, dyr, padding=1) + 1.0
+    bound = (B * H * W + 1) * 2.0 ** -24 * float(
+        torch.nn.grad.conv2d_weight(xr.abs(), wr.shape, dyr.abs(), padding=1).max() + 1.0)
+    assert float((torch_weight(dw.cpu(), 3).double() - ref_dw).abs().max()) <= bound
+
+
 # output gradients at any stride, offset and base (one value an access where
 # neither 16 nor 8 bytes are aligned), and inputs at any base
 @pytest.mark.parametrize("ks", [1, 3])
@@ -140,7 +178,7 @@ def test_weight_gradient_at_any_alignment(ks, pad, off, xshift, yshift):
 
     lib, st = P._lib(), P._stream()
     g = torch.Generator().manual_seed(100 * ks + 10 * pad + xshift + yshift)
-    B, H, W, cin, cout = 2, 9, 33, 48, 32
+    B, H, W, cin, cout = 1, 129, 131, 48, 96  # large enough for the tiled kernels
     n, ld = B * H * W, cout + pad
     xb = torch.zeros(n * cin + 8, dtype=torch.int16, device="cuda")
     yb = torch.zeros(n * ld + 8, dtype=torch.int16, device="cuda")
