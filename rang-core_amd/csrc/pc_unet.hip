@@ -595,41 +595,48 @@ __global__ __launch_bounds__(256) void k_relu_bwd(const float* __restrict__ d, i
 // levels: up 1167 -> 314 us a pass, pool 313 -> 242, pool_bwd 627 -> 392,
 // up_bwd 522 -> 517).
 template <int V>
-struct Bf16s {
-    std::uint16_t v[V];
-    __device__ __forceinline__ void load(const std::uint16_t* p) {
-        if constexpr (V == 8)
-            *reinterpret_cast<uint4*>(v) = *reinterpret_cast<const uint4*>(p);
-        else
-            v[0] = *p;
-    }
-    __device__ __forceinline__ void store(std::uint16_t* p) const {
-        if constexpr (V == 8)
-            *reinterpret_cast<uint4*>(p) = *reinterpret_cast<const uint4*>(v);
-        else
-            *p = v[0];
-    }
+struct Bf16s;
+template <>
+struct Bf16s<1> {
+    std::uint16_t v;
+    __device__ __forceinline__ void load(const std::uint16_t* p) { v = *p; }
+    __device__ __forceinline__ void store(std::uint16_t* p) const { *p = v; }
+    __device__ __forceinline__ std::uint16_t get(int) const { return v; }
+    __device__ __forceinline__ void set(int, std::uint16_t x) { v = x; }
+};
+template <>
+struct Bf16s<8> {
+    typedef std::uint16_t vec __attribute__((ext_vector_type(8)));
+    vec v;
+    __device__ __forceinline__ void load(const std::uint16_t* p) { v = *reinterpret_cast<const vec*>(p); }
+    __device__ __forceinline__ void store(std::uint16_t* p) const { *reinterpret_cast<vec*>(p) = v; }
+    __device__ __forceinline__ std::uint16_t get(int i) const { return v[i]; }
+    __device__ __forceinline__ void set(int i, std::uint16_t x) { v[i] = x; }
 };
 
 template <int V>
-struct F32s {
-    float v[V];
+struct F32s;
+template <>
+struct F32s<1> {
+    float v;
+    __device__ __forceinline__ void load(const float* p) { v = *p; }
+    __device__ __forceinline__ void store(float* p) const { *p = v; }
+    __device__ __forceinline__ float get(int) const { return v; }
+    __device__ __forceinline__ void add(int, float x) { v += x; }
+};
+template <>
+struct F32s<8> {
+    f32x4 v[2];
     __device__ __forceinline__ void load(const float* p) {
-        if constexpr (V == 8) {
-            *reinterpret_cast<float4*>(v) = *reinterpret_cast<const float4*>(p);
-            *reinterpret_cast<float4*>(v + 4) = *reinterpret_cast<const float4*>(p + 4);
-        } else {
-            v[0] = *p;
-        }
+        v[0] = *reinterpret_cast<const f32x4*>(p);
+        v[1] = *reinterpret_cast<const f32x4*>(p + 4);
     }
     __device__ __forceinline__ void store(float* p) const {
-        if constexpr (V == 8) {
-            *reinterpret_cast<float4*>(p) = *reinterpret_cast<const float4*>(v);
-            *reinterpret_cast<float4*>(p + 4) = *reinterpret_cast<const float4*>(v + 4);
-        } else {
-            *p = v[0];
-        }
+        *reinterpret_cast<f32x4*>(p) = v[0];
+        *reinterpret_cast<f32x4*>(p + 4) = v[1];
     }
+    __device__ __forceinline__ float get(int i) const { return v[i >> 2][i & 3]; }
+    __device__ __forceinline__ void add(int i, float x) { v[i >> 2][i & 3] += x; }
 };
 
 // 2 x 2 average pooling (H, W even) of C channels: BF16 in, BF16 out.
@@ -652,11 +659,11 @@ __global__ __launch_bounds__(256) void k_pool(const std::uint16_t* __restrict__ 
             Bf16s<V> t;
             t.load(x + pi * ldx + xoff + c);
 #pragma unroll
-            for (int i = 0; i < V; ++i) s[i] += from_bf16(t.v[i]);
+            for (int i = 0; i < V; ++i) s[i] += from_bf16(t.get(i));
         }
         Bf16s<V> o;
 #pragma unroll
-        for (int i = 0; i < V; ++i) o.v[i] = to_bf16(0.25f * s[i]);
+        for (int i = 0; i < V; ++i) o.set(i, to_bf16(0.25f * s[i]));
         o.store(y + po * ldy + yoff + c);
     }
 }
@@ -680,7 +687,7 @@ __global__ __launch_bounds__(256) void k_pool_bwd(const float* __restrict__ gy, 
         t.load(gy + po * ldy + yoff + c);
         o.load(gx + p * ldx + xoff + c);
 #pragma unroll
-        for (int i = 0; i < V; ++i) o.v[i] += 0.25f * t.v[i];
+        for (int i = 0; i < V; ++i) o.add(i, 0.25f * t.get(i));
         o.store(gx + p * ldx + xoff + c);
     }
 }
@@ -726,7 +733,7 @@ __global__ __launch_bounds__(256) void k_up_bwd(const float* __restrict__ gy, in
             F32s<V> t;
             t.load(gy + pi * ldy + yoff + c);
 #pragma unroll
-            for (int i = 0; i < V; ++i) s.v[i] += t.v[i];
+            for (int i = 0; i < V; ++i) s.add(i, t.get(i));
         }
         s.store(gx + po * ldx + xoff + c);
     }
