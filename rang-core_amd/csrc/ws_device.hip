@@ -514,12 +514,14 @@ __global__ __launch_bounds__(256) void k_grid_tile(const Rec* __restrict__ recs,
 // The tile side for a grid of w x h cells and kernels of ks: the largest up to
 // kTile for which the last tiles are at least ks - 1 cells wide (footprints
 // then reach at most one tile further), 0 where there is none (grids below
-// ks cells, kernels wider than a tile).
+// ks cells, kernels wider than a tile) or where a batch of layers has more tiles
+// than a launch holds workgroups.
 bool tiles(int n, int T, int ks) { return n >= ks && (n % T == 0 || n % T >= ks - 1); }
 
-int tile_side(int w, int h, int ks) {
+int tile_side(int w, int h, int ks, int batch) {
     for (int T = kTile; T >= std::max(ks, 16); --T)
-        if (tiles(w, T, ks) && tiles(h, T, ks)) return T;
+        if (tiles(w, T, ks) && tiles(h, T, ks))
+            return (long long)batch * ((w + T - 1) / T) * ((h + T - 1) / T) < (1LL << 24) ? T : 0;
     return 0;
 }
 
@@ -1087,7 +1089,7 @@ int invert(const GridInputs& i, const GridOutputs& o, double* timings, std::stri
     clear(d_sd, sizeof(double) * plane, st);
     clear(d_sp, sizeof(double) * plane, st);
     // the tiled gridding's buckets, for the batch with the most samples
-    const int tile = ks > std::size_t(kTile) ? 0 : tile_side(int(W), int(H), int(ks));
+    const int tile = ks > std::size_t(kTile) ? 0 : tile_side(int(W), int(H), int(ks), batch);
     Tiling tl{tile, 0, 0, 0};
     unsigned *d_bkey = nullptr, *d_bcnt = nullptr, *d_boff = nullptr, *d_item = nullptr, *d_ioff = nullptr, *d_sum = nullptr;
     Rec* d_rec = nullptr;
@@ -1101,7 +1103,6 @@ int invert(const GridInputs& i, const GridOutputs& o, double* timings, std::stri
             most = std::max(most, ns);
         }
         const std::size_t units = std::size_t(batch) * tl.tiles();
-        if (units >= (std::size_t(1) << 24)) throw Fail{1, "image too large for the GPU sort"};
         d_bkey = b.get<unsigned>(n);
         d_bcnt = b.get<unsigned>(4 * units + 1);
         d_boff = b.get<unsigned>(4 * units + 1);
