@@ -511,7 +511,7 @@ __global__ __launch_bounds__(256) void k_scan(DevIn in, Geo g, unsigned long lon
     for (unsigned i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) {
         if (!active<T, USE_VIS>(in, i)) continue;
         const unsigned row = row_of(g, i), ch = i - row * nchan;
-        const double w = fabs(g.fw * in.uvw[3 * row + 2] * in.foc[ch]);
+        const double w = fabs(g.fw * in.uvw[3LL * row + 2] * in.foc[ch]);
         ++cnt;
         lo = fmin(lo, w);
         hi = fmax(hi, w);
@@ -574,7 +574,7 @@ __global__ __launch_bounds__(256) void k_scan_final(const unsigned long long* bc
 // each place it (place_at rounds alike in both).
 __device__ __forceinline__ Place place_of(const DevIn& in, const Geo& g, unsigned row, unsigned ch) {
     double c[3];
-    coord_of(g, in.uvw + 3 * row, c);
+    coord_of(g, in.uvw + 3LL * row, c);
     return place_at(g, c, in.foc[ch]);
 }
 
