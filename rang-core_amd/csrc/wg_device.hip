@@ -4748,23 +4748,18 @@ int device_batch_vis2dirty(BatchImage* imgs, int n, std::size_t budget, hipStrea
             while (end < order.size() && (end == at || used + plans[order[end]].bytes <= budget))
                 used += plans[order[end++]].bytes;
             std::vector<GridPrep<T>> preps(end - at);
-            // LDS gridding; matrix-core gridding (in double precision by support)
+            // LDS gridding; matrix-core gridding, in single precision by the type of
+            // its sums, in double by support
             std::vector<GridJob<T>> jobs;
             std::map<int, std::vector<GridJob<T>>> mjobs;
             std::size_t lds = 0;
             long long total = 0;
             std::map<int, long long> mtotal;
-            // the images on the matrix cores share a launch
-            long long mvis = 0;
-            bool mdouble = false;
+            long long mvis = 0;  // visibilities of the images on the matrix cores
             int mg = 0;
-            for (std::size_t k = at; k < end; ++k) {
-                const Geo& g = plans[order[k]].g;
-                if (!g.mfma) continue;
-                mvis += g.n;
-                mdouble |= g.mfma == kMfmaDouble;
-            }
-            const int waves = grid_waves<T>(mvis, mdouble);
+            for (std::size_t k = at; k < end; ++k)
+                if (plans[order[k]].g.mfma) mvis += plans[order[k]].g.n;
+            auto waves_of = [&](const Geo& g) { return grid_waves<T>(mvis, g.mfma == kMfmaDouble); };
             for (std::size_t k = at; k < end; ++k) {
                 const int i = order[k];
                 Plan& pl = plans[i];
@@ -4774,9 +4769,9 @@ int device_batch_vis2dirty(BatchImage* imgs, int n, std::size_t budget, hipStrea
                 std::uint32_t* off;
                 sort_records<T, 0, true>(ws, pl.din, pl.g, pl.nvis, st, &recs, &off);
                 GridPrep<T>& gp = preps[k - at];
-                grid_prepare<T>(ws, pl.G, pl.g, off, 1, st, keep, timer, nullptr, gp, waves);
+                grid_prepare<T>(ws, pl.G, pl.g, off, 1, st, keep, timer, nullptr, gp, waves_of(pl.g));
                 if (gp.ub == 0) continue;
-                const int kind = sizeof(T) == 4 ? 0 : pl.g.supp;
+                const int kind = sizeof(T) == 4 ? pl.g.mfma : pl.g.supp;
                 long long& tot = pl.g.mfma ? mtotal[kind] : total;
                 if (tot + gp.ub >= (1LL << 31) || (tot + gp.ub) * 64 * gp.waves >= (1LL << 32)) throw DevError{"too many gridding items in one batch"};
                 (pl.g.mfma ? mjobs[kind] : jobs)
@@ -4811,7 +4806,9 @@ int device_batch_vis2dirty(BatchImage* imgs, int n, std::size_t budget, hipStrea
                 const GridJob<T>* d = upload(m.second);
                 const int njobs = int(m.second.size()), blocks = int(mtotal[m.first]);
                 if constexpr (sizeof(T) == 4) {
-                    const std::size_t mlds = mfma_lds<T, 1>(m.second[0].g, mg, waves);
+                    const Geo& g0 = m.second[0].g;
+                    const int waves = waves_of(g0);
+                    const std::size_t mlds = mfma_lds<T, 1>(g0, mg, waves);
                     lds_limit((const void*)k_grid_mfma_jobs<false>, mlds);
                     k_grid_mfma_jobs<false><<<blocks, 64 * waves, mlds, st>>>(d, njobs);
                     HIPCHK(hipGetLastError());
