@@ -263,7 +263,7 @@ __global__ __launch_bounds__(NT) void k_fft_rows(cx<T>* __restrict__ data, FftDe
     extern __shared__ __align__(16) unsigned char lds_raw[];
     cx<T>* buf = reinterpret_cast<cx<T>*>(lds_raw);
     cx<T>* row = data + (long long)blockIdx.x * d.n;
-    staged_fill<T, NT, MT>(buf, row, d.n, [](int e) { return std::pair<long long, int>(e, e); });
+    line_fill<T, NT, MT>(buf, row, d.n, [](int e) { return std::pair<long long, int>(e, e); });
     __syncthreads();
     fft_lds_either<T, NT, MT>(buf, d, 1, tw, sgn);
     for (int j = threadIdx.x; j < d.n; j += NT) row[j] = buf[j];
@@ -280,7 +280,7 @@ __global__ __launch_bounds__(NT) void k_fft_cols(cx<T>* __restrict__ data, int C
     const int j0 = blockIdx.x * C;
     const int nc = min(C, len - j0);
     const unsigned mnc = fft_magic(nc);
-    staged_fill<T, NT, MT>(buf, data + j0, nc * len, [&](int e) {
+    line_fill<T, NT, MT>(buf, data + j0, nc * len, [&](int e) {
         const int i = int(udiv(unsigned(e), unsigned(nc), mnc)), c = e - i * nc;
         return std::pair<long long, int>((long long)i * len + c, c * len + i);
     });
@@ -501,7 +501,7 @@ __global__ __launch_bounds__(NT) void k_ap_rows_inv(const cx<T>* __restrict__ tm
     for (int k = 0; k < nodes; ++k) {
         const double wk = w0 + double(k) * dw;
         const cx<T>* row = tmp_all + ((long long)k * n + i) * big;
-        staged_fill<T, NT, MT>(buf, row, big, [](int e) { return std::pair<long long, int>(e, e); });
+        line_fill<T, NT, MT>(buf, row, big, [](int e) { return std::pair<long long, int>(e, e); });
         __syncthreads();
         fft_lds<T, NT, MT, +1>(buf, d, 1, tw);
 #pragma unroll

@@ -551,6 +551,22 @@ __device__ __forceinline__ void staged_fill(cx<T>* buf, const cx<T>* src, int co
     }
 }
 
+// The same, or value by value for lines of 1025 to 2048 doubles: with their eight
+// values a thread staged the scheduler gives the kernel up to 236 registers, one or
+// two waves per SIMD (the surrogate's inverse rows of 2048, eight nodes, 174 -> 354
+// us; built for three waves they spill).
+template <class T, int NT, int MT, class At>
+__device__ __forceinline__ void line_fill(cx<T>* buf, const cx<T>* src, int count, At at) {
+    if constexpr (sizeof(T) == 8 && MT == 2048) {
+        for (int e = threadIdx.x; e < count; e += NT) {
+            const auto sd = at(e);
+            buf[sd.second] = src[sd.first];
+        }
+    } else {
+        staged_fill<T, NT, MT>(buf, src, count, at);
+    }
+}
+
 // Single-precision sine and cosine of `turns` whole turns: the whole turns and
 // the nearest quarter turn are taken off in double precision; what is left, at
 // most an eighth of a turn, goes through the Taylor series (first terms left
