@@ -4261,7 +4261,10 @@ void grid_prepare(Workspace& ws, const Geometry& G, const Geo& g, const std::uin
     gp.waves = g.mfma ? waves : 1;
     const int split = gp.waves > 1 ? 1 : 0;
     const std::size_t nunits = std::size_t(ntg) * (split ? 2 : 1);
-    std::uint32_t* items = static_cast<std::uint32_t*>(ws.get(kSlotItems, sizeof(std::uint32_t) * (nunits + 1)));
+    // in the fixed block they take the place of the bucket counts, which are longer
+    // and used up, so that two counts a unit need no more of it than one
+    std::uint32_t* items = static_cast<std::uint32_t*>(
+        ws.get(ws.arena ? kSlotCounts : kSlotItems, sizeof(std::uint32_t) * (nunits + 1)));
     gp.item_off = static_cast<std::uint32_t*>(ws.get(kSlotItemOff, sizeof(std::uint32_t) * (nunits + 1)));
     if (!cache || !cache->valid) {
         k_grid_items<<<(ntg + 1 + 255) / 256, 256, 0, st>>>(g, off, gp.tb.order, gp.G_planes, gp.ngroups, g.supp,
