@@ -3172,8 +3172,8 @@ void launch_degrid_mfma(int S, int nblocks, hipStream_t st, const Geo& g, const 
         k_degrid_mfma<SS><<<nblocks, 64, 0, st>>>(g, recs, off, coeff, grid, rc, item_off, order, o); \
         break;
     switch (S) {
-        DMFMA_CASE(4) DMFMA_CASE(5) DMFMA_CASE(6) DMFMA_CASE(7) DMFMA_CASE(8) DMFMA_CASE(9) DMFMA_CASE(10)
-        DMFMA_CASE(11) DMFMA_CASE(12) DMFMA_CASE(13) DMFMA_CASE(14) DMFMA_CASE(15) DMFMA_CASE(16)
+        DMFMA_CASE(7) DMFMA_CASE(8) DMFMA_CASE(9) DMFMA_CASE(10) DMFMA_CASE(11)
+        DMFMA_CASE(12) DMFMA_CASE(13) DMFMA_CASE(14) DMFMA_CASE(15) DMFMA_CASE(16)
     default:
         throw DevError{"unsupported kernel support"};
     }
@@ -3677,11 +3677,22 @@ bool fill_geo(const Geometry& G, Geo& g, int nout, bool degrid, std::string& err
     const bool single_sums = sizeof(T) == 4 && nout == 1 && g.nu % kMfmaTile == 0 && g.nv % kMfmaTile == 0;
     const bool wide = g.supp >= 6 || (g.supp == 5 && (sizeof(T) == 8 || nout == 1 || g.n >= (1LL << 20)));
     const bool fits = fixed ? single_sums : mu > 0 && mv > 0 && (degrid || single_sums || wide);
-    // degridding goes there in double precision where a tile's planes do not
-    // fit the staged LDS form (3.2 M visibilities at 1024^2, support 11: 11.6
-    // -> 4.8 ms; support 7, which fits, 1.7 ms staged and 3.0 ms there); in
-    // single precision the staged form is the faster one throughout
-    const bool unstaged = sizeof(T) == 8 && degrid_lds<T>(g.Tu, g.Tv, g.supp, P) > degrid_lds_max<T>();
+    // degridding goes there in double precision where a tile's planes do not fit
+    // the staged LDS form, from support 7 on. Stage times, a visibility per thread /
+    // here, ms: 3.2 M visibilities, support 8, 10.6 / 2.7; 116 M at support 4 on
+    // 2970^2 11 / 28, 5 on 6160^2 24 / 33, 7 on 7000^2 87 / 66, 8 and 10 on 4752^2 93 /
+    // 59 and 178 / 84; 464 M at 6 on 2376^2 120 / 162, 8 on 4752^2 307 / 228. (Staged,
+    // support 7 at 1024^2: 1.7 ms and 3.0 here; in single precision the staged form is
+    // the faster one throughout.) Where the columns of a row lie apart (transforms in
+    // two passes), the 32 x 32 cells of a product cost more than a footprint's as the
+    // data get denser, from about 2 visibilities a cell at support 12 and half as
+    // many for each one less: support 8 on 9450^2 to 11880^2, 0.3, 0.4, 0.8 and 1.3 a cell,
+    // 120 / 122, 282 / 294, 434 / 554 and 355 / 512; 10 at 0.7, 1.3 and 5.2, 877 / 839,
+    // 682 / 730 and 2079 / 2750; 12 at 0.6, 1.3 and 5.2, 1520 / 1147, 1183 / 1058 and
+    // 3493 / 4038; 13 and 15 at 0.03, 169 / 45 and 331 / 63
+    const bool sparse = double(g.n) < std::ldexp(double(g.nu) * double(g.nv), g.supp - 11);
+    const bool unstaged = sizeof(T) == 8 && g.supp >= 7 && (g.nv <= lds_fft_limit<T>() || sparse) &&
+                          degrid_lds<T>(g.Tu, g.Tv, g.supp, P) > degrid_lds_max<T>();
     g.mfma = (!degrid || unstaged) && g.wgrid && g.supp <= max_support<T>() && tile == 0 && fits && mfma_enabled()
                  ? (single_sums ? kMfmaSingle : kMfmaDouble)
                  : 0;

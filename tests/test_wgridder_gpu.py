@@ -490,3 +490,21 @@ def test_crowded_cells_keep_double_sums(nu, nv, supp):
             pairs.append([W.vis2dirty(**a, **common) for a in args])
         for first, many in pairs:
             assert rel_linf(many[inner].astype(np.float64) / n, first[inner]) < 1.2e-6
+
+
+# double-precision degridding with more planes than the staged form holds: on the
+# matrix cores from support 7 on, and, on rows transformed in two passes (8400, whose
+# columns lie apart), up to 2^(support - 11) visibilities a cell
+@pytest.mark.parametrize("supp,nu,nv,nrow", [(6, 96, 80, 400), (7, 96, 80, 400), (12, 66, 90, 400), (7, 64, 8400, 400),
+                                             (7, 64, 8400, 9000), (8, 8400, 64, 400)])
+def test_double_degridding_of_many_planes(supp, nu, nv, nrow):
+    rows = [k for k, r in enumerate(W.kernel_table()) if r[0] == supp and r[1] < 1.7]
+    kernel = (rows[len(rows) // 2], nu, nv)
+    uvw, freq, vis, wgt, nx, ny, dx = ref_case(nx=32, ny=30, field=0.5, wmax=700.0, nrow=nrow, seed=nu + supp, nchan=4)
+    x = np.random.default_rng(nv).standard_normal((nx, ny))
+    got, ref, info, rinfo = d2v(uvw, freq, x, wgt, dx, 1e-3, False, kernel=kernel)
+    same_plan(info, rinfo)
+    # 16 cells and the halo on every plane, beyond 64 KiB of LDS
+    assert (16 + supp - 1) ** 2 * info["nplanes"] * 16 > 65536
+    assert (nrow == 9000) == (nv == 8400 and info["nvis"] >= nu * nv * 2.0 ** (supp - 11))
+    assert rel_linf(got, ref) < TOL_ORACLE[False]
