@@ -303,7 +303,8 @@ struct LdsEnd {};
 // multiply-high, quarter-rate on the VALU. Several transforms recompute their
 // indices in the store phase instead, which keeps no index registers live
 // across the barrier (their kernels hold two transforms' registers).
-// The passes are bound by the VALU (97 % busy in 2048^2 column transforms), so
+// The passes are bound by the VALU and the LDS latency between (VALU issuing in 46
+// to 70 % of the SIMDs' cycles over the four 2048^2 transforms), so
 // the direction is a template argument (no sign selects) and LDS addresses step
 // by nb and ns in 32-bit additions: 16.4 -> 14.2 VALU instructions a value and
 // pass at radix 8, 24.5 -> 21.3 at radix 21.
